@@ -718,7 +718,7 @@ extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 		HIP_TRY(launch_fill_u32(sc.hist, nb, 0u, st));
 		HIP_TRY(launch_bucket_key(npoints, x, ldx, state_ids, ctx->d_state_ok, ns, ctx->dim, bb, sc.bkey, sc.hist, st));
 		HIP_TRY(launch_scan_plan(sc.hist, sc.cursor, nb, bb, ns, tables, ctx->d_cost_order, sc.plans, sc.hdr, 1,
-			ctx->dim, st));
+			ctx->dim, 0, 1, st));
 		if ((rc = stable_order(sc, npoints, nb, st))) return rc;
 		const int npass = (ctx->dt_needed + 3) / 4;
 		auto& ring = ctx->tring[1];
@@ -775,7 +775,7 @@ extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 	HIP_TRY(launch_fill_u32(sc.hist, nb, 0u, st));
 	HIP_TRY(launch_bucket_key(npoints, x, ldx, state_ids, ctx->d_state_ok, ns, ctx->dim, bb, sc.bkey, sc.hist, st));
 	HIP_TRY(launch_scan_plan(sc.hist, sc.cursor, nb, bb, ns, tables, ctx->d_cost_order, sc.plans, sc.hdr, 1,
-		ctx->dim, st));
+		ctx->dim, 0, 1, st));
 	if ((rc = stable_order(sc, npoints, nb, st))) return rc;
 
 	auto& ring = ctx->tring[1];

@@ -1,8 +1,10 @@
 // Autotuner of the sweep's formulation and launch shape, keyed by (precision,
 // D, total nodes, max dofs, log2 of the point count) and by the options that
-// restrict the candidates (formulation, waves, slab tiles). On the first forward of
+// restrict the candidates (formulation, waves, slab tiles, and through the default
+// sweep, whose kind is part of the key, the others). On the first forward of
 // a key it times every candidate on the caller's data with hipEvents and
 // keeps the fastest:
+//   * the direct or hat-table sweep, if it is the default;
 //   * the sweep where every wave walks and contracts its own block, with 2
 //     or 4 waves per workgroup and 1 or 2 dof tiles per pass (the split
 //     paths; FP64 always takes one);
@@ -33,11 +35,14 @@ int autotune(hddm_lb_ctx* ctx, int64_t npoints, const double* x, int64_t ldx, co
 		if (s && s->loaded) { nodes += s->desc.nno; maxdofs = std::max(maxdofs, s->desc.dofs); }
 	int lg = 0;
 	while (((int64_t)1 << (lg + 1)) <= npoints) lg++;
-	auto key = std::make_tuple(prec, ctx->dim, nodes, maxdofs, lg, ctx->opt_form, ctx->opt_waves, ctx->opt_slab);
+	auto key = std::make_tuple(prec, ctx->dim, nodes, maxdofs, lg, ctx->opt_form, ctx->opt_waves, ctx->opt_slab,
+		(int)cfg.kind);
 	auto hit = ctx->tuned.find(key);
 	if (hit != ctx->tuned.end()) { cfg = hit->second; ctx->tune_hits++; return HDDM_LB_SUCCESS; }
 
 	std::vector<TuneConfig> cands;
+	if (cfg.kind != TuneConfig::kWalking) cands.push_back(cfg);
+	cfg.kind = TuneConfig::kWalking;
 	if (ctx->opt_form != 2)
 		for (int waves : { 2, 4 })
 		{

@@ -322,6 +322,10 @@ extern "C" int hddm_lb_upload_state(hddm_lb_ctx* ctx, int istate, int dim, int n
 	skip_pad.resize((size_t)d.nops + kOpPad, (uint32_t)d.nops);
 	d.ops = (const Op*)up(ops_pad.data(), ops_pad.size() * sizeof(Op));
 	d.skip = (const uint32_t*)up(skip_pad.data(), skip_pad.size() * sizeof(uint32_t));
+	// as the device build: rows up to the next window are allocated and zero
+	const size_t rows = surplus_rows(nno);
+	L.s64.resize(rows * L.dofs_pad, 0.0);
+	L.s32r.resize(rows * L.dofs_pad, 0.0f);
 	d.s64 = (const double*)up(L.s64.data(), L.s64.size() * sizeof(double));
 	d.s16 = (const uint16_t*)up(L.s16.data(), L.s16.size() * sizeof(uint16_t));
 	d.sbf = (const uint16_t*)up(L.sbf.data(), L.sbf.size() * sizeof(uint16_t));
@@ -345,6 +349,13 @@ extern "C" int hddm_lb_upload_state(hddm_lb_ctx* ctx, int istate, int dim, int n
 // Installs a built state in its slot and rebuilds the descriptor tables.
 static int finish_upload(hddm_lb_ctx* ctx, int istate, int dim, std::unique_ptr<StateSlot> slot)
 {
+	auto alloc = [&](size_t bytes, int& arc) -> void* {
+		if (arc) return nullptr;
+		void* p = dev_alloc(bytes, arc);
+		if (p) slot->bufs.push_back(p);
+		return p;
+	};
+	if (int rc = build_direct_tables(slot->desc, slot->centre_exact, alloc)) return rc;
 	slot->loaded = true;
 	if ((size_t)istate >= ctx->states.size()) ctx->states.resize(istate + 1);
 	ctx->states[istate] = std::move(slot);
@@ -488,6 +499,8 @@ int prepare_tables(hddm_lb_ctx* ctx)
 	ctx->max_nseg = 1;
 	ctx->max_nseg_adj = 1;
 	ctx->nseg_adj_total = 0;
+	ctx->direct_ok = true;
+	ctx->hats_max = kHatFirst;
 	int64_t ds_offset = 0;
 	for (int s = 0; s < ns; s++)
 	{
@@ -537,11 +550,15 @@ int prepare_tables(hddm_lb_ctx* ctx)
 		ok[s] = 1;
 		ctx->dt_needed = std::max(ctx->dt_needed, d.dofs_pad / 32);
 		ctx->fmax_all = std::max(ctx->fmax_all, d.max_depth);
+		ctx->direct_ok = ctx->direct_ok && d.hats > 0;
+		ctx->hats_max = std::max(ctx->hats_max, d.hats);
 		ctx->centre_exact_all = ctx->centre_exact_all && slot.centre_exact;
 		if (d.nseg > 1) ctx->max_nseg_dp = std::max<int64_t>(ctx->max_nseg_dp, (int64_t)d.nseg * d.dofs_pad);
 		ctx->max_nseg = std::max(ctx->max_nseg, d.nseg);
 		cost.push_back(std::make_pair(-(double)d.nops / d.nseg * d.dofs_pad, s));
 	}
+	ctx->table_ok = ctx->direct_ok && ctx->hats_max <= kMaxTableHats && ctx->fmax_all <= kTabMaxFactors
+		&& sweep_table_lds_bytes(ctx->dim, ctx->hats_max, ctx->dt_needed) <= ctx->max_lds;
 	std::stable_sort(cost.begin(), cost.end());
 	std::vector<int32_t> order;
 	for (auto& c : cost) order.push_back(c.second);
@@ -620,6 +637,70 @@ int bucket_bits(int64_t npoints, int nstates, int sort)
 	return b;
 }
 
+// Which sweep a forward runs: the walking ones when a state lacks the hat
+// tables or an option asks for a formulation, launch shape or segment length
+// of theirs; the hat-table sweep when the state's hats at 64 points fit the
+// LDS (F32, FP64); the direct sweep otherwise. Each was the faster one at every
+// size measured, from 1 to 2^20 points (ms, walking / direct / hat table): D=24,
+// 128 dofs, 30,011 points F32 6.48 / 1.61 / 1.03, F16X2 5.99 / 1.61 / none; D=59,
+// 128 dofs, 16,384 points F32 32.2 / 19.7 / does not fit.
+int sweep_kind(const hddm_lb_ctx* ctx, int prec)
+{
+	if (!ctx->direct_ok || ctx->opt_form || ctx->opt_walk || ctx->opt_waves || ctx->opt_slab || ctx->opt_seg_nodes)
+		return TuneConfig::kWalking;
+	return ctx->table_ok && sweep_table_kernel_ptr(prec) ? TuneConfig::kTable : TuneConfig::kDirect;
+}
+
+// Waves per workgroup of the direct sweep: one per dof tile, at most four.
+static int direct_waves(const hddm_lb_ctx* ctx) { return std::min(ctx->dt_needed, 4); }
+
+// nt of the split (waves per workgroup; negative: the hat-table sweep's), as
+// launch_scan_plan takes it.
+static int split_waves(const hddm_lb_ctx* ctx, int kind, int prec)
+{
+	return kind == TuneConfig::kTable ? -sweep_table_waves(prec) : direct_waves(ctx);
+}
+
+// Partial elements per point of a sweep with g workgroups per block.
+static int64_t split_partial(const hddm_lb_ctx* ctx, int nt, int g)
+{
+	int64_t most = 0;
+	for (auto& s : ctx->states)
+		if (s && s->loaded)
+		{
+			const int ns = sweep_nseg(s->desc.nno, s->desc.nops, s->desc.dofs_pad / 32, nt, g);
+			if (ns > 1) most = std::max(most, (int64_t)ns * s->desc.dofs_pad);
+		}
+	return most;
+}
+
+// Workgroups per 64-point block (the nodes are split between them).
+static int split_groups(const hddm_lb_ctx* ctx, int nt, int64_t npoints)
+{
+	const int64_t nblk = (npoints + kWave - 1) / kWave;
+	int64_t g = nt < 0 ? kTableGroups / nblk : kDirectWaves / (nblk * nt);
+	g = std::max<int64_t>(1, std::min<int64_t>(g, 256));
+	// partials: at most kSplitPartialBytes, or what the walking sweeps' segments take
+	const int64_t most = std::max<int64_t>(kSplitPartialBytes, npoints * ctx->max_nseg_dp * (int64_t)sizeof(double));
+	while (g > 1 && npoints * split_partial(ctx, nt, (int)g) * (int64_t)sizeof(double) > most) g--;
+	return (int)g;
+}
+
+// FP64 elements of the segment partials of a direct or hat-table sweep of any
+// precision.
+int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints)
+{
+	int64_t most = 0;
+	for (int prec : { HDDM_LB_FP64, HDDM_LB_F32, HDDM_LB_F16X2 })
+	{
+		const int kind = sweep_kind(ctx, prec);
+		if (kind == TuneConfig::kWalking) continue;
+		const int nt = split_waves(ctx, kind, prec);
+		most = std::max(most, npoints * split_partial(ctx, nt, split_groups(ctx, nt, npoints)));
+	}
+	return most;
+}
+
 // Allocates scratch for npoints; must run outside graph capture.
 int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints)
 {
@@ -634,8 +715,11 @@ int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints)
 	if ((rc = grow(sc.cursor, sc.cap_cursor, nb))) return rc;
 	if ((rc = grow(sc.plans, sc.cap_plans, (size_t)ns))) return rc;
 	if ((rc = grow(sc.hdr, sc.cap_hdr, 1))) return rc;
-	if (ctx->max_nseg_dp > 0)
-		if ((rc = grow(sc.partial, sc.cap_partial, (size_t)npoints * (size_t)ctx->max_nseg_dp))) return rc;
+	// the tuner runs both kinds of sweep
+	size_t part = (size_t)split_partial_elems(ctx, npoints);
+	if (sweep_kind(ctx, HDDM_LB_F16X2) == TuneConfig::kWalking || ctx->opt_autotune) part = std::max(part, (size_t)npoints * (size_t)ctx->max_nseg_dp);
+	if (part > 0)
+		if ((rc = grow(sc.partial, sc.cap_partial, part))) return rc;
 	return HDDM_LB_SUCCESS;
 }
 
@@ -660,6 +744,7 @@ TuneConfig default_config(hddm_lb_ctx* ctx, int prec)
 	c.ws = ctx->opt_form == 2
 		|| (ctx->opt_form == 0 && prec == HDDM_LB_FP64 && xbanks_for(ctx->dim) == 4 && ctx->dt_needed >= 2);
 	c.nc = ctx->dt_needed >= 2 ? 4 : 2;
+	c.kind = sweep_kind(ctx, prec);
 	return c;
 }
 
@@ -675,15 +760,21 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 	const int64_t nb = (int64_t)(ns + 1) << bb;
 	HIP_TRY(launch_fill_u32(sc.hist, nb, 0u, st));
 	HIP_TRY(launch_bucket_key(npoints, x, ldx, sid, ctx->d_state_ok, ns, ctx->dim, bb, sc.bkey, sc.hist, st));
+	const bool walking = cfg.kind == TuneConfig::kWalking, table = cfg.kind == TuneConfig::kTable;
+	const int nt = walking ? 0 : split_waves(ctx, cfg.kind, prec);
+	const int groups = walking ? 1 : split_groups(ctx, nt, npoints);
 	HIP_TRY(launch_scan_plan(sc.hist, sc.cursor, nb, bb, ns, ctx->d_states, ctx->d_cost_order,
-		sc.plans, sc.hdr, !cfg.ws && cfg.walk == kWalkLds ? cfg.waves : 1, 0, st));
+		sc.plans, sc.hdr, walking && !cfg.ws && cfg.walk == kWalkLds ? cfg.waves : 1, 0, nt, groups, st));
 	HIP_TRY(launch_scatter(npoints, sc.bkey, sc.cursor, sc.perm, st));
 
-	const void* kern = cfg.ws ? sweep_ws_kernel_ptr(prec, xbanks_for(ctx->dim), ctx->fmax_all, cfg.nc)
+	const void* kern = table ? sweep_table_kernel_ptr(prec) : !walking ? sweep_direct_kernel_ptr(prec)
+		: cfg.ws ? sweep_ws_kernel_ptr(prec, xbanks_for(ctx->dim), ctx->fmax_all, cfg.nc)
 		: sweep_kernel_ptr(prec, cfg.slab, xbanks_for(ctx->dim), ctx->fmax_all, cfg.walk);
 	if (!kern) return set_error(HDDM_LB_ERROR_INVALID_VALUE, "forward: no sweep kernel for precision %d, dim %d", prec, ctx->dim);
-	const int waves = cfg.ws ? cfg.nc + 1 : cfg.waves;
-	const size_t lds = cfg.ws ? sweep_ws_lds_bytes(prec, ctx->fmax_all) : sweep_lds_bytes(prec, cfg.waves, ctx->fmax_all, cfg.walk);
+	const int waves = !walking ? std::abs(nt) : cfg.ws ? cfg.nc + 1 : cfg.waves;
+	const size_t lds = table ? sweep_table_lds_bytes(ctx->dim, ctx->hats_max, ctx->dt_needed)
+		: !walking ? sweep_direct_lds_bytes(ctx->dim, ctx->hats_max)
+		: cfg.ws ? sweep_ws_lds_bytes(prec, ctx->fmax_all) : sweep_lds_bytes(prec, cfg.waves, ctx->fmax_all, cfg.walk);
 	HIP_TRY(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 	int per_cu = 0;
 	HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, waves * kWave, lds));
@@ -691,7 +782,7 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 		return set_error(HDDM_LB_ERROR_UNSUPPORTED, "forward: sweep kernel does not fit a CU (%d waves)", waves);
 	const int grid = per_cu * ctx->num_cus;
 	// dof tiles per launch: the WS sweep's consumers cover 4 tiles (nc 4) or 1
-	const int tiles = cfg.ws ? (cfg.nc == 4 ? 4 : 1) : cfg.slab;
+	const int tiles = table ? 4 : !walking ? nt : cfg.ws ? (cfg.nc == 4 ? 4 : 1) : cfg.slab;
 
 	SweepArgs a;
 	std::memset(&a, 0, sizeof(a));
@@ -718,15 +809,16 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 	{
 		a.dt_base = sl * tiles;
 		if (sl > 0) HIP_TRY(launch_reset_counter(sc.hdr, st));
-		HIP_TRY(launch_sweep(kern, grid, waves, lds, a, st));
+		if (!walking) HIP_TRY(launch_sweep_direct(kern, grid, waves, lds, a, ctx->hats_max, st));
+		else HIP_TRY(launch_sweep(kern, grid, waves, lds, a, st));
 	}
 	if (timed)
 	{
 		HIP_TRY(hipEventRecord(ring.e1[slot], st));
 		ring.calls++;
 	}
-	if (ctx->max_nseg_dp > 0)
-		HIP_TRY(launch_reduce(ctx->d_states, sc.plans, sc.perm, sc.partial, y, ldy, ns, st));
+	if (walking ? ctx->max_nseg_dp > 0 : split_partial(ctx, nt, groups) > 0)
+		HIP_TRY(launch_reduce(ctx->d_states, sc.plans, sc.perm, sc.partial, y, ldy, ns, npoints, st));
 	return HDDM_LB_SUCCESS;
 }
 
@@ -786,9 +878,10 @@ extern "C" int hddm_lb_last_config(hddm_lb_ctx* ctx, int* config)
 {
 	if (!ctx || !config) return set_error(HDDM_LB_ERROR_INVALID_VALUE, "last_config: NULL argument");
 	const TuneConfig& c = ctx->last_cfg;
-	config[0] = c.ws ? 2 : 1;
-	config[1] = c.ws ? c.nc + 1 : c.waves;
-	config[2] = c.ws ? (c.nc == 4 ? 4 : 1) : c.slab;
+	const bool walking = c.kind == TuneConfig::kWalking, table = c.kind == TuneConfig::kTable;
+	config[0] = walking && c.ws ? 2 : 1;
+	config[1] = table ? kTableWavesF32 : !walking ? direct_waves(ctx) : c.ws ? c.nc + 1 : c.waves;
+	config[2] = table ? std::min(ctx->dt_needed, 4) : !walking ? direct_waves(ctx) : c.ws ? (c.nc == 4 ? 4 : 1) : c.slab;
 	config[3] = (int)ctx->tune_runs;
 	config[4] = (int)ctx->tune_hits;
 	return HDDM_LB_SUCCESS;

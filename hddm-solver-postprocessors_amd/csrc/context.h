@@ -92,6 +92,10 @@ struct TuneConfig
 	int ws = 0;        // 1: wave-specialized sweep (walker + consumer waves)
 	int nc = 4;        // consumer waves of the wave-specialized sweep (2 or 4)
 	int64_t seg = -1;  // node segment length used while tuning (-1: context option)
+	// kWalking: the walking sweeps, described by the fields above; kDirect, kTable:
+	// the sweeps that select nodes by hat masks (sweep_direct.hip, sweep_table.hip)
+	enum Kind { kWalking = 0, kDirect = 1, kTable = 2 };
+	int kind = kWalking;
 };
 
 } // namespace hddm_lb
@@ -122,6 +126,9 @@ struct hddm_lb_ctx
 	bool centre_exact_all = true;   // every state's StateSlot::centre_exact
 	int64_t max_nseg_dp = 0;
 	int max_nseg = 1;            // most node segments of a split state (1: none is split)
+	bool direct_ok = false;      // every state has the direct sweep's tables
+	bool table_ok = false;       // and the hat-table sweep's limits hold
+	int hats_max = 0;            // most hat ids of a state
 	hddm_lb::StateDesc* d_states = nullptr;
 	// the same descriptors with the wave-specialized adjoint's segment tables
 	hddm_lb::StateDesc* d_states_adj = nullptr;
@@ -193,7 +200,7 @@ struct hddm_lb_ctx
 	// autotuner cache: (prec, dim, total nodes, max dofs, log2 npoints) -> config
 	// (precision, D, total nodes, max dofs, log2 points, the options that
 	// restrict the candidates: formulation, waves, slab tiles)
-	std::map<std::tuple<int, int, int64_t, int, int, int, int, int>, hddm_lb::TuneConfig> tuned;
+	std::map<std::tuple<int, int, int64_t, int, int, int, int, int, int>, hddm_lb::TuneConfig> tuned;
 	int64_t tune_runs = 0, tune_hits = 0;   // keys tuned, forwards served from the cache
 	hddm_lb::TuneConfig last_cfg;           // configuration of the last eager forward
 	int last_adj[4] = { 0, 0, 0, 0 };       // hddm_lb_last_adjoint_config
@@ -211,6 +218,19 @@ int scratch_wait(hddm_lb_ctx* ctx, hipStream_t st);
 // Marks the end of an eager call's use of ctx->scratch on st.
 int scratch_mark(hddm_lb_ctx* ctx, hipStream_t st);
 int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints);
+int sweep_kind(const hddm_lb_ctx* ctx, int prec);
+int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints);
+// Waves a direct sweep, and workgroups a hat-table sweep, aim at when they
+// split a small batch's nodes. Measured (ms at 1, 2, 4, 8, 16 workgroups per
+// 64-point block): hat table, F32, D=20 / 100,005 nodes / 1,024 blocks 2.81,
+// 2.79, 2.83, 3.02, 3.53; D=24 / 12,011 nodes / 128 dofs / 469 blocks 1.08,
+// 1.04, 0.99, 1.09, 1.30; D=10 / 20,005 nodes / 11 blocks 0.46, 0.31, 0.19,
+// 0.12, 0.09. Direct, F32, D=59 / 281,077 nodes / 1,024 blocks at 2, 4, 8, 16:
+// 76.4, 70.9, 67.7, 66.8.
+constexpr int64_t kDirectWaves = 16384;
+constexpr int64_t kTableGroups = 1024;
+// Most segment partials that a split may cost.
+constexpr int64_t kSplitPartialBytes = (int64_t)32 << 20;
 TuneConfig default_config(hddm_lb_ctx* ctx, int prec);
 int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double* x, int64_t ldx,
 	const int32_t* sid, double* y, int64_t ldy, int prec, hipStream_t st, const TuneConfig& cfg, bool timed);

@@ -77,11 +77,12 @@ __global__ void __launch_bounds__(kKeyBlock) bucket_key_kernel(int64_t n, const 
 	}
 }
 
-// One workgroup of 1024 threads.
+// One workgroup of 1024 threads. dnt != 0: items and segments of the direct or
+// hat-table sweep (sweep_nseg) with dg workgroups per block.
 __global__ void __launch_bounds__(1024) scan_plan_kernel(const uint32_t* __restrict__ hist,
 	uint32_t* __restrict__ cursor, int64_t nbuckets, int bbits, int nstates,
 	const StateDesc* __restrict__ states, const int32_t* __restrict__ cost_order,
-	StatePlan* __restrict__ plans, PlanHeader* __restrict__ hdr, int group, int dxw)
+	StatePlan* __restrict__ plans, PlanHeader* __restrict__ hdr, int group, int dxw, int dnt, int dg)
 {
 	// exclusive scan of the histogram into the cursors, 1024 buckets per
 	// step with coalesced reads: a wave-level scan, then the wave totals
@@ -132,9 +133,12 @@ __global__ void __launch_bounds__(1024) scan_plan_kernel(const uint32_t* __restr
 		for (int i = 0; i < nstates; i++)
 		{
 			int s = cost_order[i];
-			int nseg = states[s].nseg;
+			const int tiles = states[s].dofs_pad >> 5;
+			const int nseg = dnt ? sweep_nseg(states[s].nno, states[s].nops, tiles, dnt, dg) : states[s].nseg;
 			plans[s].item_base = item;
-			item += (plans[s].nblk + group - 1) / group * nseg;
+			plans[s].nseg = nseg;
+			if (dnt) item += plans[s].nblk * sweep_items(nseg, tiles, dnt);
+			else item += (plans[s].nblk + group - 1) / group * nseg;
 			plans[s].partial_base = pbase;
 			plans[s].dx_base = xbase;
 			if (nseg > 1)
@@ -158,106 +162,6 @@ __global__ void scatter_kernel(int64_t n, const uint32_t* __restrict__ bkey,
 		perm[pos] = (uint32_t)p;
 	}
 }
-
-namespace {
-
-
-template <int PREC, int DT>
-__device__ __forceinline__ void contract_chunk(const SOperands<PREC, DT>& so, int ndt,
-	const double (&b)[kChunk], f16_t (&acc)[2][DT])
-{
-	if constexpr (PREC == HDDM_LB_F16X2)
-	{
-		// B is scaled by 2^12 before the split so that the low halves of
-		// basis values down to 2^-12 stay normal f16 numbers
-		uint32_t hi[8], lo[8];
-#pragma unroll
-		for (int m = 0; m < 8; m++)
-		{
-			// split in FP32 (one rounding from FP64; the f16 pair keeps 22 bits)
-			const float f0 = (float)b[2 * m] * kBScale, f1 = (float)b[2 * m + 1] * kBScale;
-			hi[m] = pack_h2(f0, f1);
-			lo[m] = pack_h2(f0 - lo_half_f16(hi[m]), f1 - hi_half_f16(hi[m]));
-		}
-		// Lanes 0-31 own points 0-31, lanes 32-63 points 32-63; each holds
-		// nodes 0-15 of its point. The B operand of points 0-31 needs nodes
-		// 0-7 in lanes 0-31 and nodes 8-15 in lanes 32-63: one half-swap.
-#pragma unroll
-		for (int m = 0; m < 4; m++)
-		{
-			auto rh = __builtin_amdgcn_permlane32_swap(hi[m], hi[m + 4], false, false);
-			hi[m] = rh[0]; hi[m + 4] = rh[1];
-			auto rl = __builtin_amdgcn_permlane32_swap(lo[m], lo[m + 4], false, false);
-			lo[m] = rl[0]; lo[m + 4] = rl[1];
-		}
-		const h8_t Bh0 = as_vec8<h8_t>(hi[0], hi[1], hi[2], hi[3]);
-		const h8_t Bh1 = as_vec8<h8_t>(hi[4], hi[5], hi[6], hi[7]);
-		const h8_t Bl0 = as_vec8<h8_t>(lo[0], lo[1], lo[2], lo[3]);
-		const h8_t Bl1 = as_vec8<h8_t>(lo[4], lo[5], lo[6], lo[7]);
-#pragma unroll
-		for (int dt = 0; dt < DT; dt++)
-			if (dt < ndt)
-			{
-				const h8_t Ah = so.A[dt][0], Al = so.A[dt][1];
-				acc[0][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Al, Bh0, acc[0][dt], 0, 0, 0);
-				acc[0][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah, Bl0, acc[0][dt], 0, 0, 0);
-				acc[0][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah, Bh0, acc[0][dt], 0, 0, 0);
-				acc[1][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Al, Bh1, acc[1][dt], 0, 0, 0);
-				acc[1][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah, Bl1, acc[1][dt], 0, 0, 0);
-				acc[1][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ah, Bh1, acc[1][dt], 0, 0, 0);
-			}
-	}
-	else if constexpr (PREC == HDDM_LB_BF16X3)
-	{
-		uint32_t t1[8], t2[8], t3[8];
-#pragma unroll
-		for (int m = 0; m < 8; m++)
-		{
-			// split in FP32: three bf16 terms carry the 24 bits of the FP32 value
-			const float f0 = (float)b[2 * m], f1 = (float)b[2 * m + 1];
-			t1[m] = pack_b2(f0, f1);
-			const float r0 = f0 - lo_half_bf16(t1[m]), r1 = f1 - hi_half_bf16(t1[m]);
-			t2[m] = pack_b2(r0, r1);
-			t3[m] = pack_b2(r0 - lo_half_bf16(t2[m]), r1 - hi_half_bf16(t2[m]));
-		}
-#pragma unroll
-		for (int m = 0; m < 4; m++)
-		{
-			auto r1 = __builtin_amdgcn_permlane32_swap(t1[m], t1[m + 4], false, false);
-			t1[m] = r1[0]; t1[m + 4] = r1[1];
-			auto r2 = __builtin_amdgcn_permlane32_swap(t2[m], t2[m + 4], false, false);
-			t2[m] = r2[0]; t2[m + 4] = r2[1];
-			auto r3 = __builtin_amdgcn_permlane32_swap(t3[m], t3[m + 4], false, false);
-			t3[m] = r3[0]; t3[m + 4] = r3[1];
-		}
-		b8_t B[2][3];
-		B[0][0] = as_vec8<b8_t>(t1[0], t1[1], t1[2], t1[3]);
-		B[1][0] = as_vec8<b8_t>(t1[4], t1[5], t1[6], t1[7]);
-		B[0][1] = as_vec8<b8_t>(t2[0], t2[1], t2[2], t2[3]);
-		B[1][1] = as_vec8<b8_t>(t2[4], t2[5], t2[6], t2[7]);
-		B[0][2] = as_vec8<b8_t>(t3[0], t3[1], t3[2], t3[3]);
-		B[1][2] = as_vec8<b8_t>(t3[4], t3[5], t3[6], t3[7]);
-#pragma unroll
-		for (int dt = 0; dt < DT; dt++)
-			if (dt < ndt)
-			{
-#pragma unroll
-				for (int t = 0; t < 2; t++)
-				{
-					// smallest products first
-					acc[t][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(so.A[dt][2], B[t][0], acc[t][dt], 0, 0, 0);
-					acc[t][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(so.A[dt][1], B[t][1], acc[t][dt], 0, 0, 0);
-					acc[t][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(so.A[dt][0], B[t][2], acc[t][dt], 0, 0, 0);
-					acc[t][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(so.A[dt][1], B[t][0], acc[t][dt], 0, 0, 0);
-					acc[t][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(so.A[dt][0], B[t][1], acc[t][dt], 0, 0, 0);
-					acc[t][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(so.A[dt][0], B[t][0], acc[t][dt], 0, 0, 0);
-				}
-			}
-	}
-}
-
-} // namespace
-
 
 // Node chunk of the walk's basis buffer: 16 nodes (the MFMA K extent) for
 // the split MFMA paths; 32 for F32, whose buffer holds floats (half as many
@@ -588,7 +492,7 @@ __global__ void __launch_bounds__(256) reduce_partials_kernel(const StateDesc* _
 	double* __restrict__ y, int64_t ldy)
 {
 	const int s = blockIdx.y;
-	const int nseg = states[s].nseg;
+	const int nseg = (int)plans[s].nseg;
 	if (nseg <= 1) return;
 	const int dofs = states[s].dofs, DP = states[s].dofs_pad;
 	const int64_t count = plans[s].count, start = plans[s].start;
@@ -676,10 +580,10 @@ hipError_t launch_bucket_key(int64_t n, const double* x, int64_t ldx, const int3
 
 hipError_t launch_scan_plan(const uint32_t* hist, uint32_t* cursor, int64_t nbuckets, int bbits, int nstates,
 	const StateDesc* states, const int32_t* cost_order, StatePlan* plans, PlanHeader* hdr, int group, int dxw,
-	hipStream_t st)
+	int dnt, int dg, hipStream_t st)
 {
 	hipLaunchKernelGGL(scan_plan_kernel, dim3(1), dim3(1024), 0, st, hist, cursor, nbuckets, bbits, nstates,
-		states, cost_order, plans, hdr, group, dxw);
+		states, cost_order, plans, hdr, group, dxw, dnt, dg);
 	return hipGetLastError();
 }
 
@@ -705,9 +609,10 @@ hipError_t launch_sweep(const void* kern, int grid, int waves, size_t lds, const
 }
 
 hipError_t launch_reduce(const StateDesc* states, const StatePlan* plans, const uint32_t* perm,
-	const double* partial, double* y, int64_t ldy, int nstates, hipStream_t st)
+	const double* partial, double* y, int64_t ldy, int nstates, int64_t npoints, hipStream_t st)
 {
-	hipLaunchKernelGGL(reduce_partials_kernel, dim3(2048, nstates), dim3(32, 8), 0, st, states, plans, perm, partial, y, ldy);
+	const int blocks = (int)(npoints < 8 * 2048 ? (npoints + 7) / 8 : 2048);
+	hipLaunchKernelGGL(reduce_partials_kernel, dim3(blocks, nstates), dim3(32, 8), 0, st, states, plans, perm, partial, y, ldy);
 	return hipGetLastError();
 }
 

@@ -81,14 +81,23 @@ hipError_t launch_bucket_key(int64_t n, const double* x, int64_t ldx, const int3
 	const uint8_t* state_ok, int nstates, int dim, int bbits, uint32_t* bkey, uint32_t* hist, hipStream_t st);
 hipError_t launch_scan_plan(const uint32_t* hist, uint32_t* cursor, int64_t nbuckets, int bbits, int nstates,
 	const StateDesc* states, const int32_t* cost_order, StatePlan* plans, PlanHeader* hdr, int group, int dxw,
-	hipStream_t st);
+	int dnt, int dg, hipStream_t st);
 hipError_t launch_scatter(int64_t n, const uint32_t* bkey, uint32_t* cursor, uint32_t* perm, hipStream_t st);
 hipError_t launch_reset_counter(PlanHeader* hdr, hipStream_t st);
 hipError_t launch_sweep(const void* kern, int grid, int waves, size_t lds, const SweepArgs& args, hipStream_t st);
 // Dynamic LDS of the sweep: the workgroup's op tiles (kWalkLds), then per
 // wave the path stack and the chunk buffer.
 size_t sweep_lds_bytes(int prec, int waves, int depth, int walk);
+// Direct sweep (sweep_direct.hip): one wave per dof tile of the pass.
+const void* sweep_direct_kernel_ptr(int prec);
+size_t sweep_direct_lds_bytes(int dim, int hats_max);
+// Hat-table sweep (sweep_table.hip), FP64 and F32 (else NULL): four dof tiles
+// per launch, sweep_table_waves waves per workgroup, launched like the direct one.
+const void* sweep_table_kernel_ptr(int prec);
+int sweep_table_waves(int prec);
+size_t sweep_table_lds_bytes(int dim, int hats_max, int tiles);
+hipError_t launch_sweep_direct(const void* kern, int grid, int waves, size_t lds, const SweepArgs& args, int hats_max, hipStream_t st);
 hipError_t launch_reduce(const StateDesc* states, const StatePlan* plans, const uint32_t* perm,
-	const double* partial, double* y, int64_t ldy, int nstates, hipStream_t st);
+	const double* partial, double* y, int64_t ldy, int nstates, int64_t npoints, hipStream_t st);
 
 } // namespace hddm_lb

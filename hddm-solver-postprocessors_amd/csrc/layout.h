@@ -2,6 +2,7 @@
 // Shared by the host library (capi.cpp, state.cpp) and the HIP kernels.
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 namespace hddm_lb {
@@ -77,7 +78,82 @@ struct StateDesc
 	const uint64_t* lomask;         // [nno] dims whose support lies in [0, 1/2]
 	const uint64_t* himask;         // [nno] dims whose support lies in [1/2, 1]
 	int64_t ds_offset;              // first element of the state's rows in an adjoint dsurplus
+	// Tables of the direct sweep (direct_tables.hip); hats == 0: the state has
+	// none and runs on the walking sweeps.
+	int hats, hstride;              // entries of hat; 16-bit ids per node in hid (2, 4, 6, 8 or 16)
+	const uint32_t* rec;            // [nodes rounded up to 64][2], see kRec*
+	const uint16_t* hid;            // [nodes rounded up to 64][hstride] 8 x the hat of each factor
+	// of the hat-table sweep, per op, rounded up to windows of 64
+	const uint32_t* trec;           // records, see kTab*
+	const uint16_t* thid;           // [hstride] 8 x the hats of the op's path
+	const int32_t* tnode;           // [windows] node of the window's first op
+	const uint32_t* hat;            // [hats][4] {LDS byte offset of the coordinate row, i, -j / i, 0} (high words)
 };
+
+// Node record of the direct sweep: word 1 is the high word of -j of the node's
+// last factor, word 0 packs the rest. i is a power of two, so the high word
+// of its FP64 value has only the top 12 bits.
+constexpr uint32_t kRecDepth2 = 0x1fu;    // twice the depth t of the last factor (P[t] is its parent product)
+constexpr uint32_t kRecPrefix = 0x20u;    // a prefix of the node is no node itself: recompute them all
+constexpr uint32_t kRecRoot = 0x40u;      // no factor: the basis is 1
+constexpr uint32_t kRecSpecial = 0x80u;   // first node of eight: one of them has one of the two bits above
+constexpr uint32_t kRecRow = 0x7e00u;     // LDS byte offset of the coordinate row (512 dim)
+constexpr uint32_t kRecIhi = 0xfff00000u;
+// The first two hat ids are no hats: no point (padding nodes) and every point
+// (padding factors).
+constexpr int kHatNone = 0;
+constexpr int kHatAll = 1;
+constexpr int kHatFirst = 2;
+// Most hats of a state: 16 KB of masks in LDS.
+constexpr int kMaxHats = 2048;
+// Record of an op in the hat-table sweep: the row of its hat in LDS (512 bytes
+// a row), twice its depth, its node's place after the window's first. The
+// empty record is the row of zeros at the deepest depth, where no product is
+// a parent's. Stored xor the empty record (0 is empty).
+constexpr uint32_t kTabRow = 0x3fe00u;
+constexpr uint32_t kTabDepth2 = 0xffu;    // alone in the low byte: GPR indexing reads that
+constexpr uint32_t kTabPrefix = 0x40000u; // the op ends no node: it has no surplus
+constexpr int kTabNodeShift = 20;
+constexpr int kMaxTableHats = 512;
+constexpr int kTabMaxFactors = 7;
+constexpr uint32_t kTabEmpty = 2u * (kTabMaxFactors - 1);
+// Waves of the hat-table sweep's workgroup (one workgroup per CU).
+constexpr int kTableWavesF32 = 12;
+constexpr int kTableWavesFP64 = 8;
+// Nodes per selection window of the direct sweep: one node per lane.
+constexpr int kWin = 64;
+
+// Allocated rows of s64 and s32r: at least one past the last node.
+constexpr size_t surplus_rows(int nno) { return ((size_t)nno / kWin + 1) * kWin; }
+// Segments of one state in the hat-table sweep with g workgroups per block
+// and nw waves each: at least a window per wave.
+constexpr int table_nseg(int nops, int nw, int g)
+{
+	const int win = (nops + kWin - 1) / kWin;
+	const int most = win < 2 * nw ? 1 : win / nw;
+	return g < most ? g : most;
+}
+// Node segments of one state in the direct sweep with nt waves per workgroup
+// and g workgroups per 64-point block: waves that a state of fewer tiles
+// leaves over take segments of their own. At least two windows a segment.
+constexpr int direct_parts(int tiles, int nt) { return tiles >= nt ? 1 : nt / tiles; }
+constexpr int direct_nseg(int nno, int tiles, int nt, int g)
+{
+	const int win = (nno + kWin - 1) / kWin;
+	const int want = g * direct_parts(tiles, nt);
+	const int most = win < 4 ? 1 : win / 2;
+	return want < most ? want : most;
+}
+// Node segments and work items per block of one state; nt > 0: the direct
+// sweep with nt waves per workgroup, nt < 0: the hat-table sweep with -nt.
+constexpr int sweep_nseg(int nno, int nops, int tiles, int nt, int g)
+{
+	return nt < 0 ? table_nseg(nops, -nt, g) : direct_nseg(nno, tiles, nt, g);
+}
+constexpr int sweep_items(int nseg, int tiles, int nt)
+{
+	return nt < 0 ? nseg : (nseg + direct_parts(tiles, nt) - 1) / direct_parts(tiles, nt);
+}
 
 // Per-state plan of one forward call, written on the device by the plan kernel.
 struct StatePlan
@@ -88,6 +164,7 @@ struct StatePlan
 	int64_t item_base;     // first work item (items ordered by state cost)
 	int64_t partial_base;  // element offset in the partial buffer (split states)
 	int64_t dx_base;       // element offset in the adjoint's dx partial buffer (split states)
+	int64_t nseg;          // node segments of the state in this call
 };
 
 struct PlanHeader

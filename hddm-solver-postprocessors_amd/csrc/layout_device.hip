@@ -476,11 +476,14 @@ int build_layout_device(int dim, int nno, int dofs,
 	out.nops = nops; out.fmax = FM; out.fstride = fstride; out.dofs_pad = DP; out.nchunks = NC;
 	out.ops = (Op*)alloc(((size_t)nops + kOpPad) * sizeof(Op), rc);
 	out.skip = (uint32_t*)alloc(((size_t)nops + kOpPad) * sizeof(uint32_t), rc);
-	out.s64 = (double*)alloc((size_t)nno * DP * sizeof(double), rc);
+	// the direct sweep loads whole groups of nodes, the hat-table sweep a row of
+	// zeros past the last: rows up to the next window are allocated and zero
+	const size_t rows = surplus_rows(nno);
+	out.s64 = (double*)alloc(rows * DP * sizeof(double), rc);
 	out.s16 = (uint16_t*)alloc((size_t)NC * 2 * DP * kChunk * sizeof(uint16_t), rc);
 	out.sbf = (uint16_t*)alloc((size_t)NC * 3 * DP * kChunk * sizeof(uint16_t), rc);
 	out.s32 = (float*)alloc((size_t)NC * DP * kChunk * sizeof(float), rc);
-	out.s32r = (float*)alloc((size_t)nno * DP * sizeof(float), rc);
+	out.s32r = (float*)alloc(rows * DP * sizeof(float), rc);
 	out.iscale = (double*)alloc((size_t)DP * sizeof(double), rc);
 	out.order = (int32_t*)alloc((size_t)nno * sizeof(int32_t), rc);
 	out.lomask = (uint64_t*)alloc((size_t)nno * sizeof(uint64_t), rc);
@@ -500,6 +503,11 @@ int build_layout_device(int dim, int nno, int dofs,
 	HDDM_DL_TRY(hipMemcpy(out.order, perm, (size_t)nno * sizeof(int32_t), hipMemcpyDeviceToDevice));
 	hipLaunchKernelGGL(masks_kernel, dim3(blocks(nno)), dim3(256), 0, st, nno, dim, (const int32_t*)d_ii,
 		(const int32_t*)d_jj, ld_index, (const uint32_t*)perm, out.lomask, out.himask);
+	if (rows > (size_t)nno)
+	{
+		HDDM_DL_TRY(hipMemset(out.s64 + (size_t)nno * DP, 0, (rows - nno) * DP * sizeof(double)));
+		HDDM_DL_TRY(hipMemset(out.s32r + (size_t)nno * DP, 0, (rows - nno) * DP * sizeof(float)));
+	}
 	HDDM_DL_TRY(hipMemset(colmax, 0, (size_t)DP * sizeof(unsigned long long)));
 	hipLaunchKernelGGL(rows_kernel, dim3(blocks((int64_t)nno * DP)), dim3(256), 0, st, nno, dofs, DP,
 		(const double*)d_S, ld_surplus, (const uint32_t*)perm, out.s64, out.s32r, colmax);

@@ -80,6 +80,13 @@ extern "C" int hddm_lb_forward_noalloc(hddm_lb_ctx* ctx, int64_t npoints,
 		return set_error(HDDM_LB_ERROR_INVALID_VALUE,
 			"forward_noalloc: %lld points need %zu bytes of scratch; at most %zu are available",
 			(long long)npoints, off, kNoAllocScratchBytes);
+	// the direct and hat-table sweeps' partials are at most kSplitPartialBytes,
+	// and only for batches small enough to be split: they fit beside the rest
+	const size_t npart = sweep_kind(ctx, precision) != TuneConfig::kWalking ? (size_t)split_partial_elems(ctx, npoints)
+		: (size_t)npoints * (size_t)ctx->max_nseg_dp;
+	if (o_part + npart * sizeof(double) > kNoAllocScratchBytes)
+		return set_error(HDDM_LB_ERROR_INVALID_VALUE, "forward_noalloc: %zu bytes of partials do not fit the scratch array",
+			npart * sizeof(double));
 	char* base = ctx->noalloc_scratch;
 	Scratch sc;
 	sc.owned = false;
@@ -89,8 +96,8 @@ extern "C" int hddm_lb_forward_noalloc(hddm_lb_ctx* ctx, int64_t npoints,
 	sc.cursor = (uint32_t*)(base + o_cursor); sc.cap_cursor = nb;
 	sc.plans = (StatePlan*)(base + o_plans); sc.cap_plans = (size_t)ns;
 	sc.hdr = (PlanHeader*)(base + o_hdr); sc.cap_hdr = 1;
-	sc.partial = ctx->max_nseg_dp > 0 ? (double*)(base + o_part) : nullptr;
-	sc.cap_partial = ctx->max_nseg_dp > 0 ? (size_t)npoints * (size_t)ctx->max_nseg_dp : 0;
+	sc.partial = npart > 0 ? (double*)(base + o_part) : nullptr;
+	sc.cap_partial = npart;
 	DeviceGuard g(ctx->device);
 	// the default launch shape: tuning would create events and time candidates
 	TuneConfig cfg = default_config(ctx, precision);

@@ -1,0 +1,67 @@
+"""GPU parity of the sweeps that pick nodes by hat masks, at the edges of their
+windows (64 nodes), groups of eight and sixteen nodes, blocks (64 points) and
+dof tiles (32), and on both sides of every rule that chooses between them.
+
+Every subset of a grid's nodes is a state, so rows drawn at random give any
+number of nodes and paths whose prefixes are no nodes. Tolerance: each of the
+nno terms B_k S_k is rounded a few times, to 53 bits (FP64) or 22 (the split
+of F16X2, the coarsest), of a term no larger than B_k max|S|: 1e-12 and 1e-6 of
+max_p sum_k B_k max|S| leave more than an order of magnitude for up to 2,000
+terms in FP64, and for the sums over them in FP32.
+"""
+import numpy as np
+import pytest
+
+import hddm_lb
+import oracle
+from gpu_util import ALL_PRECISIONS, TOL, run_forward
+
+pytestmark = pytest.mark.gpu
+
+# dim, base, depth, probability, nodes of the grid; nodes drawn (0: all); dofs; points
+CASES = [
+    (6, 3, 5, 0.0, 0, 1, 1, 1),
+    (6, 3, 5, 0.0, 0, 63, 31, 63),
+    (6, 3, 5, 0.0, 0, 64, 32, 64),
+    (6, 3, 5, 0.0, 0, 65, 33, 65),
+    (16, 2, 6, 0.3, 6000, 127, 96, 129),
+    (16, 2, 6, 0.3, 6000, 1009, 128, 700),
+    (16, 2, 6, 0.3, 6000, 1600, 160, 130),
+    (32, 2, 5, 0.3, 4000, 1024, 40, 200),
+    (59, 3, 4, 0.0, 0, 1500, 65, 100),      # more hats than the table in LDS takes
+    (10, 0, 0, 0.0, 0, 1700, 20, 90),       # up to ten factors a node
+]
+
+
+@pytest.mark.parametrize("halves", [False, True])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "d%d-n%d-c%d-p%d" % (c[0], c[5], c[6], c[7]))
+def test_node_subsets(case, halves):
+    dim, base, depth, p, nodes, pick, dofs, npts = case
+    r = np.random.default_rng(pick)
+    if depth:
+        ii, jj, lv, ix = hddm_lb.generate_grid(dim, base, depth, p, 7, nodes)
+    else:
+        hats = np.array([(0, 0), (2, 0), (2, 2), (4, 1), (4, 3)], np.int32)
+        picks = np.unique(r.integers(0, len(hats), (4 * pick, dim)) * (r.random((4 * pick, dim)) < 0.5), axis=0)
+        ii, jj = hats[picks, 0], hats[picks, 1]
+    rows = np.sort(r.choice(ii.shape[0], min(pick, ii.shape[0]), replace=False))
+    ii, jj = np.ascontiguousarray(ii[rows]), np.ascontiguousarray(jj[rows])
+    if halves:
+        # an index_i that is no power of two: these states keep the walking sweeps
+        ii, jj = np.where(ii > 1, 3 * ii, ii).astype(ii.dtype), np.where(ii > 1, 3 * jj, jj).astype(jj.dtype)
+    S = r.standard_normal((len(rows), dofs))
+    X = hddm_lb.synthetic_points(npts, dim, 9)
+    X[0] = 0.5
+    if npts > 2:
+        X[1], X[2] = 0.0, 1.0
+    yo = oracle.forward(ii, jj, S, X)
+    den = oracle.forward(ii, jj, np.ones((len(rows), 1)), X).max() * np.abs(S).max()
+    c = hddm_lb.Context(0)
+    c.upload_state(0, ii, jj, S)
+    for prec in ALL_PRECISIONS:
+        print("nodes", len(rows), "precision", prec, flush=True)
+        y = run_forward(c, X, precision=prec)
+        err = np.abs(y - yo).max() / max(den, 1e-300)
+        print("  error", err, flush=True)
+        assert err <= TOL[prec]
+    c.close()
