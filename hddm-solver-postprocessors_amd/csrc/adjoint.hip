@@ -354,12 +354,11 @@ __global__ void __launch_bounds__(256) adjoint_kernel(AdjointArgs a)
 // dx of split states: sums the node-segment partials of every point in
 // segment order. Block (64, 4): threadIdx.x walks the dims, threadIdx.y picks
 // one of 4 points; blocks stride over the state's points.
-__global__ void __launch_bounds__(256) reduce_dx_partials_kernel(const StateDesc* __restrict__ states,
-	const StatePlan* __restrict__ plans, const uint32_t* __restrict__ perm, const double* __restrict__ part,
+__global__ void __launch_bounds__(256) reduce_dx_partials_kernel(const StatePlan* __restrict__ plans, const uint32_t* __restrict__ perm, const double* __restrict__ part,
 	int dim, double* __restrict__ dx, int64_t lddx)
 {
 	const int s = blockIdx.y;
-	const int nseg = states[s].nseg;
+	const int nseg = (int)plans[s].nseg;
 	if (nseg <= 1) return;
 	const int64_t count = plans[s].count, start = plans[s].start;
 	const double* base = part + plans[s].dx_base;
@@ -479,16 +478,16 @@ using namespace hddm_lb;
 
 #define HIP_TRY(expr) do { hipError_t e_ = (expr); if (e_ != hipSuccess) return hip_fail(e_, #expr, __FILE__, __LINE__); } while (0)
 
-// After the adjoint kernels: dx of split states summed over node segments
-// (of the descriptor table the kernels used), dS summed over its copies
+// After the adjoint kernels: dx of split states summed over node segments, dS
+// summed over its copies
 // (ncopies > 1), both in a fixed order.
-static int adjoint_tail(hddm_lb_ctx* ctx, Scratch& sc, const StateDesc* tables, int max_nseg, double* dx,
+static int adjoint_tail(hddm_lb_ctx* ctx, Scratch& sc, int max_nseg, double* dx,
 	int64_t lddx, double* dsurplus, int64_t ds_total, int ncopies, int ns, hipStream_t st)
 {
 	if (dx && max_nseg > 1)
 	{
 		hipLaunchKernelGGL(reduce_dx_partials_kernel, dim3(1024, ns), dim3(64, 4), 0, st,
-			tables, (const StatePlan*)sc.plans, (const uint32_t*)sc.perm,
+			(const StatePlan*)sc.plans, (const uint32_t*)sc.perm,
 			(const double*)sc.dxpart, ctx->dim, dx, lddx);
 		HIP_TRY(hipGetLastError());
 	}
@@ -576,6 +575,16 @@ static int grow_dspart(Scratch& scr, size_t need)
 	return HDDM_LB_SUCCESS;
 }
 
+// Whether the adjoint of one-tile states at D <= 32 takes the kernels over hat
+// tables: no option asks for the per-tile ones, and the tables fit.
+static bool adjoint_table_ok(const hddm_lb_ctx* ctx)
+{
+	return sweep_kind(ctx, HDDM_LB_FP64) != TuneConfig::kWalking && ctx->dt_needed == 1 && ctx->dim <= 32
+		&& ctx->hats_max <= kMaxTableHats && ctx->fmax_all <= kTabMaxFactors
+		&& adjoint_table_lds_bytes(true, ctx->dim, ctx->hats_max) <= ctx->max_lds
+		&& adjoint_table_lds_bytes(false, ctx->dim, ctx->hats_max) <= ctx->max_lds;
+}
+
 extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 	const double* x, int64_t ldx, const int32_t* state_ids,
 	const double* gbar, int64_t ldg, double* dx, int64_t lddx,
@@ -646,7 +655,10 @@ extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 	}
 	// the wave-specialized kernel splits states into finer node segments
 	const StateDesc* tables = ws ? ctx->d_states_adj : ctx->d_states;
-	const int max_nseg = ws ? ctx->max_nseg_adj : ctx->max_nseg;
+	// one dof tile, D <= 32: the kernels over hat tables where those exist
+	const bool table = !ws && adjoint_table_ok(ctx);
+	const int groups = table ? split_groups(ctx, -adjoint_table_waves(), std::max<int64_t>(npoints, 1)) : 1;
+	const int max_nseg = table ? split_segments(ctx, -adjoint_table_waves(), groups) : ws ? ctx->max_nseg_adj : ctx->max_nseg;
 
 	// dS is accumulated: clear it with a kernel (never a memset, so the
 	// sequence stays capturable). The wave-specialized kernel adds through
@@ -736,7 +748,7 @@ extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 			HIP_TRY(hipEventRecord(ring.e1[tslot], st));
 			ring.calls++;
 		}
-		return adjoint_tail(ctx, sc, tables, max_nseg, dx, lddx, dsurplus, ds_total, ncopies, ns, st);
+		return adjoint_tail(ctx, sc, max_nseg, dx, lddx, dsurplus, ds_total, ncopies, ns, st);
 	}
 
 	// dx and dS together: the edge-sum walk for dx, then the forward's walk
@@ -744,10 +756,23 @@ extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 	int modes[2] = { dx ? kAdjDx : kAdjDs, -1 };
 	if (dx && dsurplus) modes[1] = kAdjDs;
 	const void* kerns[2] = { nullptr, nullptr };
-	int grids[2] = { 0, 0 }, groups[2] = { 0, 0 };
+	int grids[2] = { 0, 0 }, waves[2] = { 0, 0 };
 	size_t ldss[2] = { 0, 0 };
 	for (int m = 0; m < 2 && modes[m] >= 0; m++)
 	{
+		if (table)
+		{
+			const bool ds = modes[m] == kAdjDs;
+			kerns[m] = adjoint_table_kernel_ptr(ds, ctx->dim);
+			waves[m] = adjoint_table_waves();
+			ldss[m] = adjoint_table_lds_bytes(ds, ctx->dim, ctx->hats_max);
+			int per_cu = 0;
+			HIP_TRY(hipFuncSetAttribute(kerns[m], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldss[m]));
+			HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kerns[m], waves[m] * kWave, ldss[m]));
+			if (per_cu < 1) return set_error(HDDM_LB_ERROR_UNSUPPORTED, "adjoint: kernel does not fit a CU");
+			grids[m] = per_cu * ctx->num_cus;
+			continue;
+		}
 		size_t per_wave = 0;
 		const void* kern = adjoint_kernel_ptr(ctx->dim, ctx->fmax_all, modes[m], per_wave);
 		if (!kern) return set_error(HDDM_LB_ERROR_UNSUPPORTED, "adjoint: dim %d is not supported", ctx->dim);
@@ -769,13 +794,13 @@ extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 		if (bestG < 1) return set_error(HDDM_LB_ERROR_UNSUPPORTED, "adjoint: kernel does not fit a CU");
 		const size_t lds = (size_t)bestG * per_wave;
 		HIP_TRY(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-		kerns[m] = kern; grids[m] = best_per_cu * ctx->num_cus; groups[m] = bestG; ldss[m] = lds;
+		kerns[m] = kern; grids[m] = best_per_cu * ctx->num_cus; waves[m] = bestG; ldss[m] = lds;
 	}
 
 	HIP_TRY(launch_fill_u32(sc.hist, nb, 0u, st));
 	HIP_TRY(launch_bucket_key(npoints, x, ldx, state_ids, ctx->d_state_ok, ns, ctx->dim, bb, sc.bkey, sc.hist, st));
 	HIP_TRY(launch_scan_plan(sc.hist, sc.cursor, nb, bb, ns, tables, ctx->d_cost_order, sc.plans, sc.hdr, 1,
-		ctx->dim, 0, 1, st));
+		ctx->dim, table ? -adjoint_table_waves() : 0, groups, st));
 	if ((rc = stable_order(sc, npoints, nb, st))) return rc;
 
 	auto& ring = ctx->tring[1];
@@ -788,13 +813,14 @@ extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 			a.dt_base = sl;
 			if (!first) HIP_TRY(launch_reset_counter(sc.hdr, st));
 			first = false;
+			if (table) { HIP_TRY(launch_adjoint_table(kerns[m], grids[m], ldss[m], a, ctx->hats_max, st)); continue; }
 			void* params[] = { (void*)&a };
-			HIP_TRY(hipLaunchKernel(kerns[m], dim3(grids[m]), dim3(groups[m] * kWave), params, ldss[m], st));
+			HIP_TRY(hipLaunchKernel(kerns[m], dim3(grids[m]), dim3(waves[m] * kWave), params, ldss[m], st));
 		}
 	if (ctx->opt_timing)
 	{
 		HIP_TRY(hipEventRecord(ring.e1[tslot], st));
 		ring.calls++;
 	}
-	return adjoint_tail(ctx, sc, tables, max_nseg, dx, lddx, dsurplus, ds_total, ncopies, ns, st);
+	return adjoint_tail(ctx, sc, max_nseg, dx, lddx, dsurplus, ds_total, ncopies, ns, st);
 }

@@ -674,8 +674,17 @@ static int64_t split_partial(const hddm_lb_ctx* ctx, int nt, int g)
 	return most;
 }
 
+// Most node segments of a state.
+int split_segments(const hddm_lb_ctx* ctx, int nt, int g)
+{
+	int most = 1;
+	for (auto& s : ctx->states)
+		if (s && s->loaded) most = std::max(most, sweep_nseg(s->desc.nno, s->desc.nops, s->desc.dofs_pad / 32, nt, g));
+	return most;
+}
+
 // Workgroups per 64-point block (the nodes are split between them).
-static int split_groups(const hddm_lb_ctx* ctx, int nt, int64_t npoints)
+int split_groups(const hddm_lb_ctx* ctx, int nt, int64_t npoints)
 {
 	const int64_t nblk = (npoints + kWave - 1) / kWave;
 	int64_t g = nt < 0 ? kTableGroups / nblk : kDirectWaves / (nblk * nt);

@@ -219,6 +219,8 @@ int scratch_wait(hddm_lb_ctx* ctx, hipStream_t st);
 int scratch_mark(hddm_lb_ctx* ctx, hipStream_t st);
 int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints);
 int sweep_kind(const hddm_lb_ctx* ctx, int prec);
+int split_groups(const hddm_lb_ctx* ctx, int nt, int64_t npoints);
+int split_segments(const hddm_lb_ctx* ctx, int nt, int g);
 int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints);
 // Waves a direct sweep, and workgroups a hat-table sweep, aim at when they
 // split a small batch's nodes. Measured (ms at 1, 2, 4, 8, 16 workgroups per

@@ -73,6 +73,11 @@ size_t sweep_ws_lds_bytes(int prec, int depth);
 // waves; FP64 or F32; 4 dof tiles per launch. NULL when unsupported.
 const void* adjoint_ws_kernel_ptr(int prec, int xbanks, int depth);
 size_t adjoint_ws_lds_bytes(int prec, int depth, int dim, int ndx);
+// Adjoint over hat tables (adjoint_table.hip): dS or dx of one dof tile, D <= 32.
+int adjoint_table_waves();
+const void* adjoint_table_kernel_ptr(bool dsurplus, int dim);
+size_t adjoint_table_lds_bytes(bool dsurplus, int dim, int hats_max);
+hipError_t launch_adjoint_table(const void* kern, int grid, size_t lds, const AdjointArgs& args, int hats_max, hipStream_t st);
 // Register banks needed for dim (0: dim above 64 is unsupported).
 int xbanks_for(int dim);
 

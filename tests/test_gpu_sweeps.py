@@ -65,3 +65,60 @@ def test_node_subsets(case, halves):
         print("  error", err, flush=True)
         assert err <= TOL[prec]
     c.close()
+
+
+# dim, base, depth, probability, nodes of the grid; nodes drawn; dofs; points
+ADJOINT_CASES = [
+    (6, 3, 5, 0.0, 0, 1, 1, 1),
+    (6, 3, 5, 0.0, 0, 15, 16, 63),
+    (6, 3, 5, 0.0, 0, 17, 17, 64),
+    (6, 3, 5, 0.0, 0, 65, 31, 65),
+    (16, 2, 6, 0.3, 6000, 1009, 32, 700),
+    (17, 2, 5, 0.3, 4000, 1024, 5, 129),
+    (32, 2, 5, 0.3, 4000, 1500, 32, 200),
+    (10, 0, 0, 0.0, 0, 700, 20, 90),        # up to ten factors a node: the per-tile kernels
+]
+
+
+@pytest.mark.parametrize("case", ADJOINT_CASES, ids=lambda c: "d%d-n%d-c%d-p%d" % (c[0], c[5], c[6], c[7]))
+def test_adjoint_node_subsets(case):
+    """The default adjoint against the per-tile kernels' walk, at kinks too:
+    both sum the same FP64 terms in another order (1e-12 normwise for dS, whose
+    terms are products of a basis value in [0, 1] and g; 1e-10 for dx, whose
+    terms carry 1 / phi). dx is bitwise the same on every call."""
+    import torch
+    dim, base, depth, p, nodes, pick, dofs, npts = case
+    r = np.random.default_rng(pick)
+    if depth:
+        ii, jj, lv, ix = hddm_lb.generate_grid(dim, base, depth, p, 7, nodes)
+    else:
+        hats = np.array([(0, 0), (2, 0), (2, 2), (4, 1), (4, 3)], np.int32)
+        picks = np.unique(r.integers(0, len(hats), (4 * pick, dim)) * (r.random((4 * pick, dim)) < 0.5), axis=0)
+        ii, jj = hats[picks, 0], hats[picks, 1]
+    rows = np.sort(r.choice(ii.shape[0], min(pick, ii.shape[0]), replace=False))
+    ii, jj = np.ascontiguousarray(ii[rows]), np.ascontiguousarray(jj[rows])
+    S = r.standard_normal((len(rows), dofs))
+    X = hddm_lb.synthetic_points(npts, dim, 9)
+    X[0] = 0.5
+    if npts > 4:
+        X[1], X[2], X[3], X[4] = 0.0, 1.0, 1e-20, 0.25
+    x = torch.from_numpy(X).cuda()
+    g = torch.from_numpy(r.standard_normal((npts, dofs))).cuda()
+    c = hddm_lb.Context(0)
+    c.upload_state(0, ii, jj, S)
+    got = []
+    for form in (1, 0, 0):
+        c.set_option(hddm_lb.OPT_FORMULATION, form)
+        dx = torch.full((npts, dim), np.nan, dtype=torch.float64, device="cuda")
+        ds = torch.full((len(rows) * dofs,), np.nan, dtype=torch.float64, device="cuda")
+        print("nodes", len(rows), "formulation", form, flush=True)
+        c.adjoint(x, g, dx, ds, None, hddm_lb.FP64)
+        torch.cuda.synchronize()
+        assert c.device_status() == 0
+        got.append((dx.cpu().numpy(), ds.cpu().numpy()))
+    c.close()
+    (dx1, ds1), (dx0, ds0), (dxr, _) = got
+    err = [np.abs(a - b).max() / max(np.abs(b).max(), 1e-300) for a, b in ((dx0, dx1), (ds0, ds1))]
+    print("  errors", err, flush=True)
+    assert err[0] <= 1e-10 and err[1] <= 1e-12
+    assert np.array_equal(dx0, dxr)
