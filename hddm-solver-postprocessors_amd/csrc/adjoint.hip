@@ -657,8 +657,8 @@ extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 	const StateDesc* tables = ws ? ctx->d_states_adj : ctx->d_states;
 	// one dof tile, D <= 32: the kernels over hat tables where those exist
 	const bool table = !ws && adjoint_table_ok(ctx);
-	const int groups = table ? split_groups(ctx, -adjoint_table_waves(), std::max<int64_t>(npoints, 1)) : 1;
-	const int max_nseg = table ? split_segments(ctx, -adjoint_table_waves(), groups) : ws ? ctx->max_nseg_adj : ctx->max_nseg;
+	const int groups = table ? split_groups(ctx, adjoint_table_waves(), std::max<int64_t>(npoints, 1)) : 1;
+	const int max_nseg = table ? split_segments(ctx, adjoint_table_waves(), groups) : ws ? ctx->max_nseg_adj : ctx->max_nseg;
 
 	// dS is accumulated: clear it with a kernel (never a memset, so the
 	// sequence stays capturable). The wave-specialized kernel adds through
@@ -800,7 +800,7 @@ extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 	HIP_TRY(launch_fill_u32(sc.hist, nb, 0u, st));
 	HIP_TRY(launch_bucket_key(npoints, x, ldx, state_ids, ctx->d_state_ok, ns, ctx->dim, bb, sc.bkey, sc.hist, st));
 	HIP_TRY(launch_scan_plan(sc.hist, sc.cursor, nb, bb, ns, tables, ctx->d_cost_order, sc.plans, sc.hdr, 1,
-		ctx->dim, table ? -adjoint_table_waves() : 0, groups, st));
+		ctx->dim, table ? adjoint_table_waves() : 0, groups, st));
 	if ((rc = stable_order(sc, npoints, nb, st))) return rc;
 
 	auto& ring = ctx->tring[1];

@@ -500,6 +500,7 @@ int prepare_tables(hddm_lb_ctx* ctx)
 	ctx->max_nseg_adj = 1;
 	ctx->nseg_adj_total = 0;
 	ctx->direct_ok = true;
+	ctx->f32_range = true;
 	ctx->hats_max = kHatFirst;
 	int64_t ds_offset = 0;
 	for (int s = 0; s < ns; s++)
@@ -551,6 +552,7 @@ int prepare_tables(hddm_lb_ctx* ctx)
 		ctx->dt_needed = std::max(ctx->dt_needed, d.dofs_pad / 32);
 		ctx->fmax_all = std::max(ctx->fmax_all, d.max_depth);
 		ctx->direct_ok = ctx->direct_ok && d.hats > 0;
+		ctx->f32_range = ctx->f32_range && d.f32_range;
 		ctx->hats_max = std::max(ctx->hats_max, d.hats);
 		ctx->centre_exact_all = ctx->centre_exact_all && slot.centre_exact;
 		if (d.nseg > 1) ctx->max_nseg_dp = std::max<int64_t>(ctx->max_nseg_dp, (int64_t)d.nseg * d.dofs_pad);
@@ -559,6 +561,7 @@ int prepare_tables(hddm_lb_ctx* ctx)
 	}
 	ctx->table_ok = ctx->direct_ok && ctx->hats_max <= kMaxTableHats && ctx->fmax_all <= kTabMaxFactors
 		&& sweep_table_lds_bytes(ctx->dim, ctx->hats_max, ctx->dt_needed) <= ctx->max_lds;
+	ctx->direct_ok = ctx->direct_ok && (ctx->table_ok || sweep_direct_lds_bytes(ctx->dim, ctx->hats_max) <= ctx->max_lds);
 	std::stable_sort(cost.begin(), cost.end());
 	std::vector<int32_t> order;
 	for (auto& c : cost) order.push_back(c.second);
@@ -640,25 +643,31 @@ int bucket_bits(int64_t npoints, int nstates, int sort)
 // Which sweep a forward runs: the walking ones when a state lacks the hat
 // tables or an option asks for a formulation, launch shape or segment length
 // of theirs; the hat-table sweep when the state's hats at 64 points fit the
-// LDS (F32, FP64); the direct sweep otherwise. Each was the faster one at every
-// size measured, from 1 to 2^20 points (ms, walking / direct / hat table): D=24,
-// 128 dofs, 30,011 points F32 6.48 / 1.61 / 1.03, F16X2 5.99 / 1.61 / none; D=59,
-// 128 dofs, 16,384 points F32 32.2 / 19.7 / does not fit.
+// LDS; the direct sweep otherwise.
+// The last two compute in FP64 or in F32. A split precision takes F32 there:
+// with the basis formed once for many nodes the F32 MFMAs cost less than
+// forming the split operands, and every product is exact to 24 bits instead
+// of 22. Measured (ms, walking / split operands in a direct sweep / F32):
+// F16X2 at D=24, 128 dofs, 30,011 points 5.99 / 1.61 / 1.07, at D=59, 128 dofs,
+// 16,384 points 30.0 / 16.2 / 16.0; F32 there 6.49 and 32.5 walking.
+// It needs surpluses that F32 holds; states with a dof column whose largest
+// value lies outside 2^-100 .. 2^100 keep the walking sweeps, whose f16
+// operands are scaled by column.
 int sweep_kind(const hddm_lb_ctx* ctx, int prec)
 {
 	if (!ctx->direct_ok || ctx->opt_form || ctx->opt_walk || ctx->opt_waves || ctx->opt_slab || ctx->opt_seg_nodes)
 		return TuneConfig::kWalking;
-	return ctx->table_ok && sweep_table_kernel_ptr(prec) ? TuneConfig::kTable : TuneConfig::kDirect;
+	if ((prec == HDDM_LB_F16X2 || prec == HDDM_LB_BF16X3) && !ctx->f32_range) return TuneConfig::kWalking;
+	return ctx->table_ok ? TuneConfig::kTable : TuneConfig::kDirect;
 }
 
-// Waves per workgroup of the direct sweep: one per dof tile, at most four.
-static int direct_waves(const hddm_lb_ctx* ctx) { return std::min(ctx->dt_needed, 4); }
+// The precision that the direct and hat-table sweeps compute in.
+static int sweep_prec(int prec) { return prec == HDDM_LB_FP64 ? HDDM_LB_FP64 : HDDM_LB_F32; }
 
-// nt of the split (waves per workgroup; negative: the hat-table sweep's), as
-// launch_scan_plan takes it.
-static int split_waves(const hddm_lb_ctx* ctx, int kind, int prec)
+// Waves per workgroup of a direct or hat-table sweep.
+static int split_waves(int kind, int prec)
 {
-	return kind == TuneConfig::kTable ? -sweep_table_waves(prec) : direct_waves(ctx);
+	return kind == TuneConfig::kTable ? sweep_table_waves(sweep_prec(prec)) : kDirectWaves;
 }
 
 // Partial elements per point of a sweep with g workgroups per block.
@@ -668,7 +677,7 @@ static int64_t split_partial(const hddm_lb_ctx* ctx, int nt, int g)
 	for (auto& s : ctx->states)
 		if (s && s->loaded)
 		{
-			const int ns = sweep_nseg(s->desc.nno, s->desc.nops, s->desc.dofs_pad / 32, nt, g);
+			const int ns = sweep_nseg(s->desc.nops, nt, g);
 			if (ns > 1) most = std::max(most, (int64_t)ns * s->desc.dofs_pad);
 		}
 	return most;
@@ -679,7 +688,7 @@ int split_segments(const hddm_lb_ctx* ctx, int nt, int g)
 {
 	int most = 1;
 	for (auto& s : ctx->states)
-		if (s && s->loaded) most = std::max(most, sweep_nseg(s->desc.nno, s->desc.nops, s->desc.dofs_pad / 32, nt, g));
+		if (s && s->loaded) most = std::max(most, sweep_nseg(s->desc.nops, nt, g));
 	return most;
 }
 
@@ -687,8 +696,7 @@ int split_segments(const hddm_lb_ctx* ctx, int nt, int g)
 int split_groups(const hddm_lb_ctx* ctx, int nt, int64_t npoints)
 {
 	const int64_t nblk = (npoints + kWave - 1) / kWave;
-	int64_t g = nt < 0 ? kTableGroups / nblk : kDirectWaves / (nblk * nt);
-	g = std::max<int64_t>(1, std::min<int64_t>(g, 256));
+	int64_t g = std::max<int64_t>(1, std::min<int64_t>(kSplitGroups / nblk, 256));
 	// partials: at most kSplitPartialBytes, or what the walking sweeps' segments take
 	const int64_t most = std::max<int64_t>(kSplitPartialBytes, npoints * ctx->max_nseg_dp * (int64_t)sizeof(double));
 	while (g > 1 && npoints * split_partial(ctx, nt, (int)g) * (int64_t)sizeof(double) > most) g--;
@@ -700,11 +708,11 @@ int split_groups(const hddm_lb_ctx* ctx, int nt, int64_t npoints)
 int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints)
 {
 	int64_t most = 0;
-	for (int prec : { HDDM_LB_FP64, HDDM_LB_F32, HDDM_LB_F16X2 })
+	for (int prec : { HDDM_LB_FP64, HDDM_LB_F32 })
 	{
 		const int kind = sweep_kind(ctx, prec);
 		if (kind == TuneConfig::kWalking) continue;
-		const int nt = split_waves(ctx, kind, prec);
+		const int nt = split_waves(kind, prec);
 		most = std::max(most, npoints * split_partial(ctx, nt, split_groups(ctx, nt, npoints)));
 	}
 	return most;
@@ -770,17 +778,17 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 	HIP_TRY(launch_fill_u32(sc.hist, nb, 0u, st));
 	HIP_TRY(launch_bucket_key(npoints, x, ldx, sid, ctx->d_state_ok, ns, ctx->dim, bb, sc.bkey, sc.hist, st));
 	const bool walking = cfg.kind == TuneConfig::kWalking, table = cfg.kind == TuneConfig::kTable;
-	const int nt = walking ? 0 : split_waves(ctx, cfg.kind, prec);
+	const int nt = walking ? 0 : split_waves(cfg.kind, prec);
 	const int groups = walking ? 1 : split_groups(ctx, nt, npoints);
 	HIP_TRY(launch_scan_plan(sc.hist, sc.cursor, nb, bb, ns, ctx->d_states, ctx->d_cost_order,
 		sc.plans, sc.hdr, walking && !cfg.ws && cfg.walk == kWalkLds ? cfg.waves : 1, 0, nt, groups, st));
 	HIP_TRY(launch_scatter(npoints, sc.bkey, sc.cursor, sc.perm, st));
 
-	const void* kern = table ? sweep_table_kernel_ptr(prec) : !walking ? sweep_direct_kernel_ptr(prec)
+	const void* kern = table ? sweep_table_kernel_ptr(sweep_prec(prec)) : !walking ? sweep_direct_kernel_ptr(sweep_prec(prec))
 		: cfg.ws ? sweep_ws_kernel_ptr(prec, xbanks_for(ctx->dim), ctx->fmax_all, cfg.nc)
 		: sweep_kernel_ptr(prec, cfg.slab, xbanks_for(ctx->dim), ctx->fmax_all, cfg.walk);
 	if (!kern) return set_error(HDDM_LB_ERROR_INVALID_VALUE, "forward: no sweep kernel for precision %d, dim %d", prec, ctx->dim);
-	const int waves = !walking ? std::abs(nt) : cfg.ws ? cfg.nc + 1 : cfg.waves;
+	const int waves = !walking ? nt : cfg.ws ? cfg.nc + 1 : cfg.waves;
 	const size_t lds = table ? sweep_table_lds_bytes(ctx->dim, ctx->hats_max, ctx->dt_needed)
 		: !walking ? sweep_direct_lds_bytes(ctx->dim, ctx->hats_max)
 		: cfg.ws ? sweep_ws_lds_bytes(prec, ctx->fmax_all) : sweep_lds_bytes(prec, cfg.waves, ctx->fmax_all, cfg.walk);
@@ -791,7 +799,7 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 		return set_error(HDDM_LB_ERROR_UNSUPPORTED, "forward: sweep kernel does not fit a CU (%d waves)", waves);
 	const int grid = per_cu * ctx->num_cus;
 	// dof tiles per launch: the WS sweep's consumers cover 4 tiles (nc 4) or 1
-	const int tiles = table ? 4 : !walking ? nt : cfg.ws ? (cfg.nc == 4 ? 4 : 1) : cfg.slab;
+	const int tiles = !walking ? 4 : cfg.ws ? (cfg.nc == 4 ? 4 : 1) : cfg.slab;
 
 	SweepArgs a;
 	std::memset(&a, 0, sizeof(a));
@@ -889,8 +897,8 @@ extern "C" int hddm_lb_last_config(hddm_lb_ctx* ctx, int* config)
 	const TuneConfig& c = ctx->last_cfg;
 	const bool walking = c.kind == TuneConfig::kWalking, table = c.kind == TuneConfig::kTable;
 	config[0] = walking && c.ws ? 2 : 1;
-	config[1] = table ? kTableWavesF32 : !walking ? direct_waves(ctx) : c.ws ? c.nc + 1 : c.waves;
-	config[2] = table ? std::min(ctx->dt_needed, 4) : !walking ? direct_waves(ctx) : c.ws ? (c.nc == 4 ? 4 : 1) : c.slab;
+	config[1] = table ? kTableWavesF32 : !walking ? kDirectWaves : c.ws ? c.nc + 1 : c.waves;
+	config[2] = !walking ? std::min(ctx->dt_needed, 4) : c.ws ? (c.nc == 4 ? 4 : 1) : c.slab;
 	config[3] = (int)ctx->tune_runs;
 	config[4] = (int)ctx->tune_hits;
 	return HDDM_LB_SUCCESS;

@@ -129,6 +129,7 @@ struct hddm_lb_ctx
 	bool direct_ok = false;      // every state has the direct sweep's tables
 	bool table_ok = false;       // and the hat-table sweep's limits hold
 	int hats_max = 0;            // most hat ids of a state
+	bool f32_range = false;      // every state's surpluses are in F32's range
 	hddm_lb::StateDesc* d_states = nullptr;
 	// the same descriptors with the wave-specialized adjoint's segment tables
 	hddm_lb::StateDesc* d_states_adj = nullptr;
@@ -222,15 +223,12 @@ int sweep_kind(const hddm_lb_ctx* ctx, int prec);
 int split_groups(const hddm_lb_ctx* ctx, int nt, int64_t npoints);
 int split_segments(const hddm_lb_ctx* ctx, int nt, int g);
 int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints);
-// Waves a direct sweep, and workgroups a hat-table sweep, aim at when they
-// split a small batch's nodes. Measured (ms at 1, 2, 4, 8, 16 workgroups per
-// 64-point block): hat table, F32, D=20 / 100,005 nodes / 1,024 blocks 2.81,
-// 2.79, 2.83, 3.02, 3.53; D=24 / 12,011 nodes / 128 dofs / 469 blocks 1.08,
-// 1.04, 0.99, 1.09, 1.30; D=10 / 20,005 nodes / 11 blocks 0.46, 0.31, 0.19,
-// 0.12, 0.09. Direct, F32, D=59 / 281,077 nodes / 1,024 blocks at 2, 4, 8, 16:
-// 76.4, 70.9, 67.7, 66.8.
-constexpr int64_t kDirectWaves = 16384;
-constexpr int64_t kTableGroups = 1024;
+// Workgroups that a direct or hat-table sweep aims at when it splits a small
+// batch's nodes. Measured (ms at 1, 2, 4, 8, 16 workgroups per 64-point block):
+// hat table, F32, D=20 / 100,005 nodes / 1,024 blocks 2.81, 2.79, 2.83, 3.02,
+// 3.53; D=24 / 12,011 nodes / 128 dofs / 469 blocks 1.08, 1.04, 0.99, 1.09, 1.30;
+// D=10 / 20,005 nodes / 11 blocks 0.46, 0.31, 0.19, 0.12, 0.09.
+constexpr int64_t kSplitGroups = 1024;
 // Most segment partials that a split may cost.
 constexpr int64_t kSplitPartialBytes = (int64_t)32 << 20;
 TuneConfig default_config(hddm_lb_ctx* ctx, int prec);

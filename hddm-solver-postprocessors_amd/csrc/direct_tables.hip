@@ -21,6 +21,7 @@ struct HatTable
 	uint32_t id[kHashSlots];
 	int total;                            // hats found
 	int overflow;                         // a key found no slot
+	int wide;                             // a dof column's largest value is out of F32's range
 };
 
 // i is a power of two: its exponent, the dim and the centre name the hat.
@@ -39,7 +40,7 @@ __device__ __forceinline__ uint32_t hat_slot(unsigned long long key)
 __global__ void direct_init_kernel(HatTable* t)
 {
 	for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < kHashSlots; s += gridDim.x * blockDim.x) t->key[s] = 0ull;
-	if (blockIdx.x == 0 && threadIdx.x == 0) { t->total = 0; t->overflow = 0; }
+	if (blockIdx.x == 0 && threadIdx.x == 0) { t->total = 0; t->overflow = 0; t->wide = 0; }
 }
 
 // Padding nodes: phi = max(0, 1 - |0 x - 2|) = 0.
@@ -104,12 +105,15 @@ __global__ void hat_insert_kernel(int64_t nent, const uint32_t* __restrict__ fta
 	t->overflow = 1;
 }
 
-// One workgroup of 1024 threads: ids in slot order, and the hats' records.
-__global__ void __launch_bounds__(1024) hat_number_kernel(HatTable* t, uint32_t* __restrict__ hat)
+// One workgroup of 1024 threads: ids in slot order, the hats' records, and
+// whether the columns' largest values (2^14 to 2^15 iscale) lie in 2^-100 .. 2^100.
+__global__ void __launch_bounds__(1024) hat_number_kernel(HatTable* t, uint32_t* __restrict__ hat, int DP, const double* __restrict__ iscale)
 {
 	__shared__ int wsum[16];
 	constexpr int kPer = kHashSlots / 1024;
 	const int tid = threadIdx.x, lane = tid & 63;
+	for (int c = tid; c < DP; c += 1024)
+		if (iscale[c] < 0x1p-114 || iscale[c] > 0x1p+85) t->wide = 1;
 	int mine = 0;
 	for (int k = 0; k < kPer; k++) mine += t->key[tid * kPer + k] != 0ull;
 	int x = mine;
@@ -232,13 +236,13 @@ int build_direct_tables(StateDesc& d, bool centre_exact, const DeviceAlloc& allo
 	hipLaunchKernelGGL(prefix_kernel, dim3(grid_for((int64_t)d.nops * kWave)), dim3(256), 0, st, d.nno, d.nops, d.ops, rec);
 	hipLaunchKernelGGL(special_kernel, dim3(grid_for(npad / 8)), dim3(256), 0, st, d.nno, npad, rec);
 	hipLaunchKernelGGL(hat_insert_kernel, dim3(grid_for(nent)), dim3(256), 0, st, nent, d.ftab, t);
-	hipLaunchKernelGGL(hat_number_kernel, dim3(1), dim3(1024), 0, st, t, hat);
+	hipLaunchKernelGGL(hat_number_kernel, dim3(1), dim3(1024), 0, st, t, hat, d.dofs_pad, d.iscale);
 	hipLaunchKernelGGL(hat_lookup_kernel, dim3(grid_for((int64_t)npad * hs)), dim3(256), 0, st, d.nno, npad, fs, hs, d.ftab,
 		(const HatTable*)t, hid);
 	hipLaunchKernelGGL(table_rec_kernel, dim3(grid_for(qpad)), dim3(256), 0, st, d.nops, qpad, hs, d.ops, (const uint16_t*)hid, trec,
 		thid, tnode);
 	HIP_TRY(hipGetLastError());
-	int found[2] = { 0, 0 };
+	int found[3] = { 0, 0, 0 };
 	HIP_TRY(hipMemcpy(found, &t->total, sizeof(found), hipMemcpyDeviceToHost));
 	if (found[1] || found[0] > kMaxHats) return HDDM_LB_SUCCESS;
 	d.rec = rec;
@@ -248,6 +252,7 @@ int build_direct_tables(StateDesc& d, bool centre_exact, const DeviceAlloc& allo
 	d.hid = hid;
 	d.hat = hat;
 	d.hstride = hs;
+	d.f32_range = !found[2];
 	d.hats = found[0];
 	return HDDM_LB_SUCCESS;
 }

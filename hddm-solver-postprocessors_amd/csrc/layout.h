@@ -81,6 +81,7 @@ struct StateDesc
 	// Tables of the direct sweep (direct_tables.hip); hats == 0: the state has
 	// none and runs on the walking sweeps.
 	int hats, hstride;              // entries of hat; 16-bit ids per node in hid (2, 4, 6, 8 or 16)
+	int f32_range;                  // largest value of every dof column 0 or within 2^-100 .. 2^100
 	const uint32_t* rec;            // [nodes rounded up to 64][2], see kRec*
 	const uint16_t* hid;            // [nodes rounded up to 64][hstride] 8 x the hat of each factor
 	// of the hat-table sweep, per op, rounded up to windows of 64
@@ -120,41 +121,21 @@ constexpr uint32_t kTabEmpty = 2u * (kTabMaxFactors - 1);
 // Waves of the hat-table sweep's workgroup (one workgroup per CU).
 constexpr int kTableWavesF32 = 12;
 constexpr int kTableWavesFP64 = 8;
+// Waves of the direct sweep's.
+constexpr int kDirectWaves = 8;
 // Nodes per selection window of the direct sweep: one node per lane.
 constexpr int kWin = 64;
 
 // Allocated rows of s64 and s32r: at least one past the last node.
 constexpr size_t surplus_rows(int nno) { return ((size_t)nno / kWin + 1) * kWin; }
-// Segments of one state in the hat-table sweep with g workgroups per block
-// and nw waves each: at least a window per wave.
-constexpr int table_nseg(int nops, int nw, int g)
+// Segments of one state in the direct and hat-table sweeps with g workgroups
+// per block and nw waves each: at least a window per wave.
+constexpr int sweep_nseg(int nops, int nw, int g)
 {
 	const int win = (nops + kWin - 1) / kWin;
 	const int most = win < 2 * nw ? 1 : win / nw;
 	return g < most ? g : most;
 }
-// Node segments of one state in the direct sweep with nt waves per workgroup
-// and g workgroups per 64-point block: waves that a state of fewer tiles
-// leaves over take segments of their own. At least two windows a segment.
-constexpr int direct_parts(int tiles, int nt) { return tiles >= nt ? 1 : nt / tiles; }
-constexpr int direct_nseg(int nno, int tiles, int nt, int g)
-{
-	const int win = (nno + kWin - 1) / kWin;
-	const int want = g * direct_parts(tiles, nt);
-	const int most = win < 4 ? 1 : win / 2;
-	return want < most ? want : most;
-}
-// Node segments and work items per block of one state; nt > 0: the direct
-// sweep with nt waves per workgroup, nt < 0: the hat-table sweep with -nt.
-constexpr int sweep_nseg(int nno, int nops, int tiles, int nt, int g)
-{
-	return nt < 0 ? table_nseg(nops, -nt, g) : direct_nseg(nno, tiles, nt, g);
-}
-constexpr int sweep_items(int nseg, int tiles, int nt)
-{
-	return nt < 0 ? nseg : (nseg + direct_parts(tiles, nt) - 1) / direct_parts(tiles, nt);
-}
-
 // Per-state plan of one forward call, written on the device by the plan kernel.
 struct StatePlan
 {

@@ -1,50 +1,53 @@
-// Direct sweep of the LinearBasis forward (gfx950).
+// Direct sweep of the LinearBasis forward (gfx950), F32 and FP64, for states
+// whose hats do not fit the LDS as a table of values.
 //
-// One workgroup takes one 64-point block against one range of the state's
-// nodes (trie order); each of its waves contracts one 32-dof tile (waves that
-// a narrow state leaves over take ranges of their own). Per item:
+// One workgroup of eight waves takes one 64-point block against one range of
+// the state's nodes (trie order) and up to four 32-dof tiles. Per item:
 //   1. the block's coordinates go to LDS, one row of 64 per dimension;
 //   2. every distinct hat of the state (a few hundred) is evaluated once at
 //      the block's points; the 64-bit mask of the points inside its support
 //      goes to LDS;
-//   3. one node per lane, the masks of a node's hats are ANDed: the node is
-//      alive if a point is left. 64 nodes cost a few loads and a ballot,
-//      where a walk that tests prefix products visits them one by one;
-//   4. the alive nodes' basis values are formed, one point per lane, in trie
+//   3. the waves take windows of 64 nodes in turn. One node per lane, the
+//      masks of a node's hats are ANDed: the node is alive if a point is
+//      left. 64 nodes cost a few loads and a ballot, where a walk that tests
+//      prefix products visits them one by one;
+//   4. in rounds, every wave forms the basis of a part of its window (32
+//      nodes in F32, 16 in FP64: 8 KB) into LDS, one point per lane, in trie
 //      order: P[t + 1] = P[t] * phi, the prefix products in registers under
-//      GPR indexing (a node's parents are nodes before it, alive when it
-//      is). Each value is an MFMA operand as it stands.
-// Nothing in 4. decides which node comes next, so records and surplus rows
-// of the next eight nodes load while eight are computed, and the eight hats
-// are independent of each other.
+//      GPR indexing (a node's parents are nodes before it, alive when it is);
+//   5. every wave contracts one dof tile against the basis of its share of
+//      the waves. F32 and FP64 MFMAs run on the vector unit itself, so the
+//      basis, some 75 issue cycles a node against the MFMA's 64 (F32) or 128
+//      (FP64), is formed once for all tiles and not once per tile;
+//   6. the sums of waves of one tile are added through LDS, in order.
 //
 // Contraction, one wave, 64 points x 32 dofs:
-//   F32   v_mfma_f32_32x32x1_2b_f32: one node per step, the two blocks of
-//         which are the two halves of the 64 points, so lane p holds the B
+//   F32   v_mfma_f32_32x32x1_2b_f32: one alive node per step, the two blocks
+//         of which are the two halves of the 64 points, so lane p holds the B
 //         operand of point p as the basis was formed; folded into FP64 after
 //         every 32 nodes of the layout;
-//   FP64  v_mfma_f64_16x16x4f64: four nodes per step, brought from one point
-//         per lane to its layout by two rounds of row swaps; a 16-point
-//         column tile where all four nodes are zero is skipped;
-//   F16X2, BF16X3  as the walking sweep, 16 nodes per step.
-// Groups of nodes and folds are fixed by the layout, and what is skipped is
-// exactly zero, so a point's result does not depend on the points it shares
-// a block with.
+//   FP64  v_mfma_f64_16x16x4f64: four nodes per step, read from LDS in its
+//         operand layout; a 16-point column tile where all four nodes are
+//         zero is skipped.
+// Groups of nodes, folds and which wave adds which are fixed by the layout,
+// and what is skipped is exactly zero, so a point's result does not depend on
+// the points it shares a block with.
 //
-// Measured against the walking sweeps (ms, before -> here): D=59 / 281,077
-// nodes / 128 dofs / 16,384 points F32 32.3 -> 19.7, FP64 82.1 -> 27.8; D=24 /
-// 12,011 nodes / 128 dofs / 30,011 points F16X2 6.0 -> 1.6, BF16X3 7.3 -> 1.8.
-// At D=59 some 70 % of the nodes meet a point of any block, so nearly every
-// node costs its hat, its product and its MFMAs: the vector unit's issue.
+// Measured (ms; walking sweeps -> every wave forming the basis of its own tile
+// -> here): D=59 / 281,077 nodes / 128 dofs / 16,384 points F32 32.5 -> 19.7 ->
+// 16.0, FP64 82.3 -> 27.8 -> 21.8. At D=59 some 70 % of the nodes meet a point
+// of any block; the MFMAs of those are 5.3 ms of the F32 time.
 #include "sweep_common.h"
 #include "kernels.h"
-#include "contract.h"
 
 #include <type_traits>
 
 namespace hddm_lb {
 
 namespace {
+
+constexpr int kDW = kDirectWaves;
+constexpr int kBasisBytes = 8192;               // per wave
 
 typedef double dv4_t __attribute__((ext_vector_type(4)));
 typedef float fv32_t __attribute__((ext_vector_type(32)));
@@ -106,27 +109,28 @@ __device__ __forceinline__ double hat(double x, double i, double nj)
 // hat, and so its basis, is zero at every point.
 constexpr uint32_t kFarHigh = 0xfe37e43cu;
 
-// The surplus operands of a unit of kU nodes and its contraction.
+// The contraction of a unit of eight nodes.
 template <int PREC> struct Contract;
 
 template <>
 struct Contract<HDDM_LB_F32>
 {
-	static constexpr int kU = 8;
 	typedef float B;                // basis values as the contraction takes them
+	static constexpr int kSub = 32; // nodes per wave and round
+	static constexpr int kAcc = 32;
 	struct S { float v[8]; };
 	fv32_t acc;
-	double acc64[32];
+	double sum[32];
 	int chunk;                      // 32-node chunk acc sums
 	const float* base;
 	int off[8];
 
-	__device__ __forceinline__ void init(const StateDesc* sd, int DP, int tile, int lane, int n0)
+	__device__ __forceinline__ void init(const StateDesc* sd, int DP, int tile, int lane)
 	{
 #pragma unroll
-		for (int r = 0; r < 32; r++) acc64[r] = 0.0;
+		for (int r = 0; r < 32; r++) sum[r] = 0.0;
 		zero();
-		chunk = n0 >> 5;
+		chunk = -1;
 		base = ldc(&sd->s32r) + 32 * tile;
 #pragma unroll
 		for (int k = 0; k < 8; k++) off[k] = k * DP + (lane & 31);
@@ -151,57 +155,51 @@ struct Contract<HDDM_LB_F32>
 	__device__ __forceinline__ void fold()
 	{
 #pragma unroll
-		for (int r = 0; r < 32; r++) acc64[r] += (double)acc[r];
+		for (int r = 0; r < 32; r++) sum[r] += (double)acc[r];
 	}
 
 	__device__ __forceinline__ void begin(int n0)
 	{
 		if ((n0 >> 5) != chunk)
 		{
-			fold();
-			zero();
+			if (chunk >= 0) { fold(); zero(); }
 			chunk = n0 >> 5;
 		}
 	}
 
-	__device__ __forceinline__ void contract(const S& s, const float (&b)[8])
+	// the unit's basis: rows of 64 points
+	__device__ __forceinline__ void contract(const S& s, const B* basis, uint32_t mask, int lane)
 	{
+		float b[8];
 #pragma unroll
-		for (int k = 0; k < 8; k++) acc = __builtin_amdgcn_mfma_f32_32x32x1f32(s.v[k], b[k], acc, 0, 0, 0);
+		for (int k = 0; k < 8; k++) b[k] = basis[k * kWave + lane];
+#pragma unroll
+		for (int k = 0; k < 8; k++)
+			if ((mask >> k) & 1u) acc = __builtin_amdgcn_mfma_f32_32x32x1f32(s.v[k], b[k], acc, 0, 0, 0);
 	}
 
-	__device__ __forceinline__ void finish(const StateDesc*, int, int) { fold(); }
+	__device__ __forceinline__ void finish() { fold(); }
+	__device__ __forceinline__ double get(int r) const { return sum[r]; }
 
 	// D of v_mfma_f32_32x32x1_2b: block t in registers 16 t .., register r
 	// of lane l holds row 8 (r / 4) + 4 (l / 32) + r % 4 (the dof) and column
-	// l % 32 (the point).
-	template <typename F>
-	__device__ __forceinline__ void store(F out, int lane)
-	{
-#pragma unroll
-		for (int t = 0; t < 2; t++)
-		{
-			double v[16];
-#pragma unroll
-			for (int r = 0; r < 16; r++) v[r] = acc64[16 * t + r];
-			out(32 * t + (lane & 31), lane, v);
-		}
-	}
-	static constexpr bool kRows32 = true;
+	// l % 32 (the point)
+	__device__ __forceinline__ static int point(int i, int lane) { return 32 * (i >> 4) + (lane & 31); }
+	__device__ __forceinline__ static int dof(int i, int lane) { return 8 * ((i & 15) >> 2) + 4 * (lane >> 5) + (i & 3); }
 };
 
 template <>
 struct Contract<HDDM_LB_FP64>
 {
-	static constexpr int kU = 8;
 	typedef double B;
+	static constexpr int kSub = 16;
+	static constexpr int kAcc = 32;
 	struct S { double v[2][2]; };   // [quad][16-dof half]: S[node 4 q + lane / 16][dof 16 h + lane % 16]
 	dv4_t acc[2][4];                // [16-dof half][16-point tile]
-
 	const double* base;
 	int off;
 
-	__device__ __forceinline__ void init(const StateDesc* sd, int DP, int tile, int lane, int)
+	__device__ __forceinline__ void init(const StateDesc* sd, int DP, int tile, int lane)
 	{
 #pragma unroll
 		for (int h = 0; h < 2; h++)
@@ -221,138 +219,53 @@ struct Contract<HDDM_LB_FP64>
 	}
 
 	__device__ __forceinline__ void begin(int) {}
-	__device__ __forceinline__ static void swap32(double& a, double& b)
-	{
-		auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
-		auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
-		a = __hiloint2double((int)hi[0], (int)lo[0]);
-		b = __hiloint2double((int)hi[1], (int)lo[1]);
-	}
 
-	__device__ __forceinline__ static void swap16(double& a, double& b)
+	__device__ __forceinline__ void contract(const S& s, const B* basis, uint32_t mask, int lane)
 	{
-		auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
-		auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
-		a = __hiloint2double((int)hi[0], (int)lo[0]);
-		b = __hiloint2double((int)hi[1], (int)lo[1]);
-	}
-
-	__device__ __forceinline__ void contract(const S& s, const double (&bv)[8])
-	{
+		const double* row = basis + (lane >> 4) * kWave + (lane & 15);
 #pragma unroll
 		for (int q = 0; q < 2; q++)
-		{
-			double b0 = bv[4 * q], b1 = bv[4 * q + 1], b2 = bv[4 * q + 2], b3 = bv[4 * q + 3];
-			const uint64_t nz = __builtin_amdgcn_ballot_w64((b0 != 0.0) | (b1 != 0.0) | (b2 != 0.0) | (b3 != 0.0));
-			if (nz)
+			if ((mask >> (4 * q)) & 15u)
 			{
-				// rows of 16 lanes: from [node][row = point tile] to [point tile][row = node]
-				swap32(b0, b2);
-				swap32(b1, b3);
-				swap16(b0, b1);
-				swap16(b2, b3);
-				const double b[4] = { b0, b1, b2, b3 };
+				double b[4];
+#pragma unroll
+				for (int p = 0; p < 4; p++) b[p] = row[4 * q * kWave + 16 * p];
 #pragma unroll
 				for (int p = 0; p < 4; p++)
-					if ((nz >> (16 * p)) & 0xffffull)
+					if (__builtin_amdgcn_ballot_w64(b[p] != 0.0))
 					{
 						acc[0][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(s.v[q][0], b[p], acc[0][p], 0, 0, 0);
 						acc[1][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(s.v[q][1], b[p], acc[1][p], 0, 0, 0);
 					}
 			}
-		}
 	}
 
-	__device__ __forceinline__ void finish(const StateDesc*, int, int) {}
-	static constexpr bool kRows32 = false;
+	__device__ __forceinline__ void finish() {}
+	__device__ __forceinline__ double get(int r) const { return acc[r >> 4][(r >> 2) & 3][r & 3]; }
+
+	// D[i][j] in lane j + 16 (i % 4), element i / 4: i the dof, j the point
+	__device__ __forceinline__ static int point(int i, int lane) { return 16 * ((i >> 2) & 3) + (lane & 15); }
+	__device__ __forceinline__ static int dof(int i, int lane) { return 16 * (i >> 4) + 4 * (i & 3) + (lane >> 4); }
 };
-
-// F16X2 and BF16X3: the operand split and products of the walking sweep.
-template <int PREC>
-struct ContractSplit
-{
-	static constexpr int kU = 16;
-	static constexpr int kTerms = PREC == HDDM_LB_F16X2 ? 2 : 3;
-	typedef float B;
-	typedef SOperands<PREC, 1> S;
-	double acc64[2][16];
-	const uint16_t* base;           // rows of 16 nodes: [chunk][term][dof][16]
-	int off;
-
-	__device__ __forceinline__ void init(const StateDesc* sd, int, int tile, int lane, int)
-	{
-#pragma unroll
-		for (int t = 0; t < 2; t++)
-#pragma unroll
-			for (int r = 0; r < 16; r++) acc64[t][r] = 0.0;
-		base = (PREC == HDDM_LB_F16X2 ? ldc(&sd->s16) : ldc(&sd->sbf)) + 32 * tile * kChunk;
-		off = (lane & 31) * kChunk + (lane >> 5) * 8;
-	}
-
-	__device__ __forceinline__ void load(S& s, int n0, int DP)
-	{
-		const uint16_t* sc = base + (size_t)(n0 >> 4) * kTerms * DP * kChunk;
-#pragma unroll
-		for (int t = 0; t < kTerms; t++, sc += (size_t)DP * kChunk) s.A[0][t] = *(const typename S::V*)(sc + off);
-	}
-
-	__device__ __forceinline__ void begin(int) {}
-
-	__device__ __forceinline__ void contract(const S& s, const float (&b)[16])
-	{
-		f16_t acc[2][1];
-#pragma unroll
-		for (int t = 0; t < 2; t++)
-#pragma unroll
-			for (int r = 0; r < 16; r++) acc[t][0][r] = 0.0f;
-		contract_chunk<PREC, 1>(s, 1, b, acc);
-#pragma unroll
-		for (int t = 0; t < 2; t++)
-#pragma unroll
-			for (int r = 0; r < 16; r++) acc64[t][r] += (double)acc[t][0][r];
-	}
-
-	__device__ __forceinline__ void finish(const StateDesc* sd, int tile, int lane)
-	{
-		if constexpr (PREC == HDDM_LB_F16X2)
-		{
-			const double* iscale = ldc(&sd->iscale) + 32 * tile + 4 * (lane >> 5);
-#pragma unroll
-			for (int r = 0; r < 16; r++)
-			{
-				const double f = iscale[8 * (r >> 2) + (r & 3)] * (1.0 / kBScale);
-				acc64[0][r] *= f;
-				acc64[1][r] *= f;
-			}
-		}
-	}
-
-	template <typename F>
-	__device__ __forceinline__ void store(F out, int lane)
-	{
-#pragma unroll
-		for (int t = 0; t < 2; t++) out(32 * t + (lane & 31), lane, acc64[t]);
-	}
-	static constexpr bool kRows32 = true;
-};
-template <> struct Contract<HDDM_LB_F16X2> : ContractSplit<HDDM_LB_F16X2> {};
-template <> struct Contract<HDDM_LB_BF16X3> : ContractSplit<HDDM_LB_BF16X3> {};
 
 } // namespace
 
 template <int PREC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) sweep_direct_kernel(SweepArgs a, int hats_max)
+__global__ void __launch_bounds__(64 * kDW) __attribute__((amdgpu_waves_per_eu(2))) sweep_direct_kernel(SweepArgs a, int hats_max)
 {
 	extern __shared__ __attribute__((aligned(16))) double lds[];
 	typedef Contract<PREC> C;
-	constexpr int U = C::kU;
-	constexpr uint64_t UM = ((uint64_t)1 << U) - 1;
+	typedef typename C::B B;
+	constexpr int U = 8, kUnits = C::kSub / U;              // units per wave and round
+	constexpr uint32_t kSubMask = C::kSub == 32 ? ~0u : (1u << C::kSub) - 1u;
 	const int lane = threadIdx.x & 63;
 	const int wave = uniform((int)(threadIdx.x >> 6));
-	const int nt = uniform((int)(blockDim.x >> 6));
-	char* const xl = (char*)lds + lane * 8;                 // the lane's column of the coordinate rows
-	uint64_t* const M = (uint64_t*)(lds + (size_t)a.dim * kWave);
+	B* const basis = (B*)lds;                               // [wave][node of the round][point]
+	double* const X = lds + kDW * kBasisBytes / 8;
+	char* const xl = (char*)X + lane * 8;                   // the lane's column of the coordinate rows
+	uint64_t* const M = (uint64_t*)(X + (size_t)a.dim * kWave);
 	int64_t* const slot = (int64_t*)(M + hats_max);
+	uint8_t* const alive = (uint8_t*)(slot + 1);            // [wave][unit]: a round's alive nodes
 	const int64_t nitems = ldc(&a.hdr->nitems);
 
 	for (;;)
@@ -370,16 +283,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) s
 			const int si = ldc(&a.cost_order[i]);
 			const int64_t ib = ldc(&a.plans[si].item_base);
 			const int64_t nb = ldc(&a.plans[si].nblk);
-			const int parts = direct_parts(ldc(&a.states[si].dofs_pad) >> 5, nt);
-			const int64_t ng = (ldc(&a.plans[si].nseg) + parts - 1) / parts;
-			if (item < ib + nb * ng) { s = si; local = item - ib; nblk = nb; break; }
+			if (item < ib + nb * ldc(&a.plans[si].nseg)) { s = si; local = item - ib; nblk = nb; break; }
 		}
 		const StateDesc* sd = a.states + s;
 		const StatePlan* pl = a.plans + s;
-		const int64_t group = local / nblk, blk = local - group * nblk;
+		const int64_t seg = local / nblk, blk = local - seg * nblk;
 		const int dofs = ldc(&sd->dofs), DP = ldc(&sd->dofs_pad);
 		const int nno = ldc(&sd->nno);
-		const int nseg = (int)ldc(&pl->nseg);
 		const int tiles = DP >> 5;
 		if (a.dt_base >= tiles) continue;
 		const int64_t start = ldc(&pl->start) + blk * kWave, count = ldc(&pl->count);
@@ -387,7 +297,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) s
 		const int np = rem < kWave ? (int)rem : kWave;
 		const uint32_t orig = a.perm[start + (lane < np ? lane : np - 1)];
 		const double* xrow = a.x + (int64_t)orig * a.ldx;
-		for (int d = wave; d < a.dim; d += nt) *(double*)(xl + d * (kWave * 8)) = xrow[d];
+		for (int d = wave; d < a.dim; d += kDW) *(double*)(xl + d * (kWave * 8)) = xrow[d];
 		__syncthreads();
 		// the points inside each hat's support
 		{
@@ -396,14 +306,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) s
 			const uint64_t valid = np < kWave ? ((uint64_t)1 << np) - 1 : ~(uint64_t)0;
 			if (threadIdx.x == 0) { M[kHatAll] = valid; M[kHatNone] = 0; }
 			// four hats at a time (the last group repeats its first hat)
-			for (int h = kHatFirst + wave; h < hats; h += 4 * nt)
+			for (int h = kHatFirst + wave; h < hats; h += 4 * kDW)
 			{
 				uint64_t in[4];
 				int at[4];
 #pragma unroll
 				for (int j = 0; j < 4; j++)
 				{
-					at[j] = h + j * nt < hats ? h + j * nt : h;
+					at[j] = h + j * kDW < hats ? h + j * kDW : h;
 					const u4_t e = ldc(ht + at[j]);
 					const double u = (*(const double*)(xl + e[0]) + f64_from_high(e[2])) * f64_from_high(e[1]);
 					in[j] = __builtin_amdgcn_ballot_w64(fmax(1.0 - fabs(u), 0.0) > 0.0) & valid;
@@ -417,12 +327,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) s
 		}
 		__syncthreads();
 
-		const int tl = tiles < nt ? tiles : nt;
-		const int part = wave / tl, tile = a.dt_base + wave - part * tl;
-		const int seg = (int)group * direct_parts(tiles, nt) + part;
-		if (part >= direct_parts(tiles, nt) || seg >= nseg || tile >= tiles) continue;
+		// the wave's tile, and the waves whose basis it contracts
+		const int tw = min(tiles - a.dt_base, 4);
+		const int parts = kDW / tw;
+		const int part = wave / tw, tile = a.dt_base + wave - part * tw;
+		const bool on = part < parts;
+		const int f0 = kDW * part / parts, f1 = kDW * (part + 1) / parts;
 		const int nwin = (nno + kWin - 1) / kWin;
-		const int w0 = (int)((int64_t)nwin * seg / nseg), w1 = (int)((int64_t)nwin * (seg + 1) / nseg);
+		const int nseg = (int)ldc(&pl->nseg);
+		const int s0 = (int)((int64_t)nwin * seg / nseg), s1 = (int)((int64_t)nwin * (seg + 1) / nseg);
+		const int turns = (s1 - s0 + kDW - 1) / kDW;        // windows s0 + wave + kDW i
 
 		const uv16_t* const recs = (const uv16_t*)ldc(&sd->rec);
 		const u4_t* const ftab = (const u4_t*)ldc(&sd->ftab);
@@ -442,24 +356,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) s
 			}
 			return p;
 		};
-		if (w0 > 0)
-		{
-			const uint32_t r0 = ldc((const uint32_t*)recs + (size_t)w0 * kWin * 2);
-			if (!(r0 & kRecRoot)) (void)path(w0 * kWin, (int)((r0 & kRecDepth2) >> 1));
-		}
 		C c;
-		c.init(sd, DP, tile, lane, w0 * kWin);
-		uint32_t st_nodes = 0, st_chunks = 0, st_mfma = 0;
+		c.init(sd, DP, tile, lane);
 
-		for (int wb = w0; wb < w1; wb += kWave)
+		for (int tb = 0; tb < turns; tb += kWave)
 		{
-			// selection: the alive nodes of window wb + i as lane i of (mlo, mhi)
-			const int nb = min(kWave, w1 - wb);
+			// selection: the alive nodes of the wave's window of turn tb + i as
+			// lane i of (mlo, mhi)
+			const int first = s0 + wave + tb * kDW;
+			const int nb = min(kWave, (s1 - first + kDW - 1) / kDW);   // <= 0: no window
 			uint32_t mlo = 0, mhi = 0;
 			auto select = [&](auto words) {
 				constexpr int W = decltype(words)::value;   // pairs of hat ids per node
 				constexpr int kSel = 16 / W < 8 ? 16 / W : 8;   // windows in flight
-				const uint32_t* hid = (const uint32_t*)ldc(&sd->hid) + ((size_t)wb * kWin + lane) * W;
+				const uint32_t* hid = (const uint32_t*)ldc(&sd->hid) + ((size_t)first * kWin + lane) * W;
 #pragma unroll 1
 				for (int i = 0; i < nb; i += kSel)
 				{
@@ -467,7 +377,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) s
 #pragma unroll
 					for (int j = 0; j < kSel; j++)
 					{
-						const uint32_t* src = hid + (size_t)min(i + j, nb - 1) * kWin * W;
+						const uint32_t* src = hid + (size_t)(min(i + j, nb - 1) * kDW) * (kWin * W);
 #pragma unroll
 						for (int w = 0; w < W; w++) id[j][w] = src[w];
 					}
@@ -479,7 +389,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) s
 						for (int w = 0; w < W; w++)
 							m &= *(const uint64_t*)((const char*)M + (id[j][w] & 0xffffu)) & *(const uint64_t*)((const char*)M + (id[j][w] >> 16));
 						const uint64_t al = __builtin_amdgcn_ballot_w64(m != 0);
-						// lanes nb .. are never read as windows
 						if (lane == i + j && i + j < nb)
 						{
 							mlo = (uint32_t)al;
@@ -496,175 +405,182 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) s
 			case 8: select(std::integral_constant<int, 4>()); break;
 			default: select(std::integral_constant<int, 8>()); break;
 			}
-
-			// Units of U nodes with a node alive; while one is computed the next
-			// one's surplus rows and records load. Records come through the
-			// scalar cache, out of order with LDS reads, so they are requested
-			// only after the unit's coordinates have been read: a wait for
-			// those would wait for the records too.
-			struct Unit { int n0; uint32_t mask; uv16_t rec[U / 8]; };
-			uint64_t wm = __builtin_amdgcn_ballot_w64((mlo | mhi) != 0u), m64 = 0;
-			int cw = 0;
-			auto next = [&](Unit& u) -> bool {
-				if (!m64)
-				{
-					if (!wm) return false;
-					cw = __builtin_ctzll(wm);
-					wm &= wm - 1;
-					m64 = ((uint64_t)__builtin_amdgcn_readlane(mhi, cw) << 32) | (uint32_t)__builtin_amdgcn_readlane(mlo, cw);
-				}
-				const int o = __builtin_ctzll(m64) & ~(U - 1);
-				u.mask = (uint32_t)((m64 >> o) & UM);
-				m64 &= ~(UM << o);
-				u.n0 = (wb + cw) * kWin + o;
-#pragma unroll
-				for (int r = 0; r < U / 8; r++) u.rec[r] = ldc(recs + (size_t)(u.n0 >> 3) + r);
-				return true;
-			};
-			Unit u;
-			typename C::S su;
-			bool more = next(u);
-			if (more) c.load(su, u.n0, DP);
-#pragma unroll 1
-			while (more)
-			{
-				double x[U];
-#pragma unroll
-				for (int k = 0; k < U; k++) x[k] = *(const double*)(xl + (u.rec[k / 8][2 * (k % 8)] & kRecRow));
-				__builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
-				__builtin_amdgcn_sched_barrier(0);
-				Unit v = u;
-				typename C::S sv;
-				more = next(v);
-				c.load(sv, v.n0, DP);
-				__builtin_amdgcn_sched_barrier(0);
-				c.begin(u.n0);
-				typename C::B b[U];
-				// all hats before the products: independent chains
-#pragma unroll
-				for (int k = 0; k < U; k++)
-				{
-					const uint32_t r0 = u.rec[k / 8][2 * (k % 8)], r1 = u.rec[k / 8][2 * (k % 8) + 1];
-					x[k] = hat(x[k], f64_from_high(r0 & kRecIhi), f64_from_high((u.mask >> k) & 1u ? r1 : kFarHigh));
-				}
-				uint32_t special = 0;
-#pragma unroll
-				for (int r = 0; r < U / 8; r++) special |= u.rec[r][0];
-				if (special & kRecSpecial)
-				{
-					// rare: the root, or a node with a prefix that is no node;
-					// the whole path of every node
-#pragma unroll
-					for (int k = 0; k < U; k++) b[k] = (typename C::B)0;
-#pragma unroll 1
-					for (uint32_t m = u.mask; m; m &= m - 1)
-					{
-						const int k = __builtin_ctz(m);
-						const uint32_t r0 = ldc((const uint32_t*)recs + 2 * (size_t)(u.n0 + k));
-						const double p = path(u.n0 + k, r0 & kRecRoot ? 0 : (int)((r0 & kRecDepth2) >> 1) + 1);
-#pragma unroll
-						for (int j = 0; j < U; j++) b[j] = k == j ? (typename C::B)p : b[j];
-					}
-				}
-				else
-				{
-#pragma unroll
-					for (int k = 0; k < U; k += 4)
-					{
-						const uv16_t& r = u.rec[k / 8];
-						const int j = 2 * (k % 8);
-						mulp4(P, r[j], r[j + 2], r[j + 4], r[j + 6], x[k], x[k + 1], x[k + 2], x[k + 3],
-							b[k], b[k + 1], b[k + 2], b[k + 3]);
-					}
-				}
-				c.contract(su, b);
-				u = v;
-				su = sv;
-			}
 			if (a.stats)
 			{
-				// counted in a pass of its own (statistics mode only)
-				uint32_t alive = (uint32_t)__popc(mlo) + (uint32_t)__popc(mhi);
-				uint32_t ch = PREC == HDDM_LB_F32 ? (mlo != 0u) + (mhi != 0u) : 0u;
-				if constexpr (PREC != HDDM_LB_F32)
-					for (int o = 0; o < 32; o += U) ch += (((mlo >> o) & (uint32_t)UM) != 0u) + (((mhi >> o) & (uint32_t)UM) != 0u);
+				// statistics mode: alive nodes, their chunks (F32) or units
+				// (FP64), F32 MFMAs
+				uint32_t nodes = (uint32_t)__popc(mlo) + (uint32_t)__popc(mhi), ch = 0;
+				for (int o = 0; o < 32; o += C::kSub == 32 ? 32 : U)
+				{
+					const uint32_t um = C::kSub == 32 ? ~0u : 0xffu << o;
+					ch += ((mlo & um) != 0u) + ((mhi & um) != 0u);
+				}
 				for (int off = 32; off; off >>= 1)
 				{
-					alive += __shfl_xor(alive, off, 64);
+					nodes += __shfl_xor(nodes, off, 64);
 					ch += __shfl_xor(ch, off, 64);
 				}
-				st_nodes += alive;
-				st_chunks += ch;
-				st_mfma += PREC == HDDM_LB_F32 ? alive : (PREC == HDDM_LB_F16X2 ? 6u * ch : (PREC == HDDM_LB_BF16X3 ? 12u * ch : 0u));
-			}
-		}
-
-		c.finish(sd, tile, lane);
-		const bool split = nseg > 1;
-		double* const part_s = a.partial + ldc(&pl->partial_base) + ((int64_t)seg * count + blk * kWave) * DP;
-		if constexpr (C::kRows32)
-			c.store([&](int qp, int ln, const double (&v)[16]) {
-				const uint32_t oq = (uint32_t)__shfl((int)orig, qp, 64);
-				if (qp < np)
+				if (lane == 0)
 				{
-					double* out = split ? part_s + (int64_t)qp * DP : a.y + (int64_t)oq * a.ldy;
-#pragma unroll
-					for (int r = 0; r < 16; r++)
+					atomicAdd(&a.stats[0], (unsigned long long)nodes);
+					atomicAdd(&a.stats[2], (unsigned long long)ch);
+					if (PREC == HDDM_LB_F32) atomicAdd(&a.stats[4], (unsigned long long)nodes * tw);
+				}
+			}
+
+			const int rounds = min(kWave, turns - tb) * (kWin / C::kSub);
+			bool ahead = false;                             // the products above the window are there
+#pragma unroll 1
+			for (int r = 0; r < rounds; r++)
+			{
+				const int i = r / (kWin / C::kSub), sub = r % (kWin / C::kSub);
+				const uint64_t m64 = ((uint64_t)__builtin_amdgcn_readlane(mhi, i) << 32) | (uint32_t)__builtin_amdgcn_readlane(mlo, i);
+				const uint32_t mask = (uint32_t)(m64 >> (sub * C::kSub)) & kSubMask;
+				const int wn = (first + i * kDW) * kWin, n0 = wn + sub * C::kSub;
+				if (sub == 0) ahead = false;
+				if (tw > 1) __syncthreads();                // the round before has been contracted
+				else __builtin_amdgcn_wave_barrier();
+				if (lane < kUnits) alive[wave * kUnits + lane] = (uint8_t)(mask >> (8 * lane));
+				if (mask)
+				{
+					if (!ahead)
 					{
-						const int dof = 32 * tile + 8 * (r >> 2) + 4 * (ln >> 5) + (r & 3);
-						if (dof < dofs) out[dof] = v[r];
+						const uint32_t r0 = ldc((const uint32_t*)recs + (size_t)wn * 2);
+						if (!(r0 & kRecRoot)) (void)path(wn, (int)((r0 & kRecDepth2) >> 1));
+						ahead = true;
+					}
+					// Units with a node alive; while one is computed the next one's
+					// records load. Those come through the scalar cache, out of
+					// order with LDS reads, so they are requested only after the
+					// unit's coordinates have been read: a wait for those would
+					// wait for the records too.
+					uint32_t left = mask;
+					int o = __builtin_ctz(left) & ~(U - 1);
+					uv16_t rec = ldc(recs + (size_t)((n0 + o) >> 3));
+#pragma unroll 1
+					for (;;)
+					{
+						const uint32_t um = (left >> o) & 0xffu;
+						left &= ~(0xffu << o);
+						double x[U];
+#pragma unroll
+						for (int k = 0; k < U; k++) x[k] = *(const double*)(xl + (rec[2 * k] & kRecRow));
+						__builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+						__builtin_amdgcn_sched_barrier(0);
+						const int no = left ? __builtin_ctz(left) & ~(U - 1) : o;
+						const uv16_t nrec = ldc(recs + (size_t)((n0 + no) >> 3));
+						__builtin_amdgcn_sched_barrier(0);
+						B* const out = basis + (size_t)(wave * C::kSub + o) * kWave + lane;
+						B b[U];
+						if (rec[0] & kRecSpecial)
+						{
+							// rare: the root, or a node with a prefix that is no node;
+							// the whole path of every node
+#pragma unroll
+							for (int k = 0; k < U; k++) b[k] = (B)0;
+#pragma unroll 1
+							for (uint32_t m = um; m; m &= m - 1)
+							{
+								const int k = __builtin_ctz(m);
+								const uint32_t r0 = ldc((const uint32_t*)recs + 2 * (size_t)(n0 + o + k));
+								const double p = path(n0 + o + k, r0 & kRecRoot ? 0 : (int)((r0 & kRecDepth2) >> 1) + 1);
+#pragma unroll
+								for (int j = 0; j < U; j++) b[j] = k == j ? (B)p : b[j];
+							}
+						}
+						else
+						{
+							// all hats before the products: independent chains
+#pragma unroll
+							for (int k = 0; k < U; k++)
+								x[k] = hat(x[k], f64_from_high(rec[2 * k] & kRecIhi), f64_from_high((um >> k) & 1u ? rec[2 * k + 1] : kFarHigh));
+#pragma unroll
+							for (int k = 0; k < U; k += 4)
+								mulp4(P, rec[2 * k], rec[2 * k + 2], rec[2 * k + 4], rec[2 * k + 6], x[k], x[k + 1], x[k + 2], x[k + 3],
+									b[k], b[k + 1], b[k + 2], b[k + 3]);
+						}
+#pragma unroll
+						for (int k = 0; k < U; k++) out[k * kWave] = b[k];
+						if (!left) break;
+						o = no;
+						rec = nrec;
 					}
 				}
-			}, lane);
-		else
-		{
-			// D[i][j] in lane j + 16 (i % 4), element i / 4: i the dof, j the point
-#pragma unroll
-			for (int p = 0; p < 4; p++)
-			{
-				const int qp = 16 * p + (lane & 15);
-				const uint32_t oq = (uint32_t)__shfl((int)orig, qp, 64);
-				if (qp < np)
+				if (tw > 1) __syncthreads();                // the round's basis is there
+				else __builtin_amdgcn_wave_barrier();
+				if (!on) continue;
+				// The units of this wave's share, in node order; while one is
+				// contracted the next one's surplus rows load.
+				const uint32_t av = lane < (f1 - f0) * kUnits ? alive[f0 * kUnits + lane] : 0u;
+				uint64_t units = __builtin_amdgcn_ballot_w64(av != 0u);
+				if (!units) continue;
+				const int wfirst = s0 + f0 + (tb + i) * kDW;
+				int j = __builtin_ctzll(units);
+				auto node = [&](int u) { return (wfirst + u / kUnits) * kWin + sub * C::kSub + (u % kUnits) * U; };
+				typename C::S sb;
+				c.load(sb, node(j), DP);
+#pragma unroll 1
+				for (;;)
 				{
-					double* out = split ? part_s + (int64_t)qp * DP : a.y + (int64_t)oq * a.ldy;
-#pragma unroll
-					for (int h = 0; h < 2; h++)
-#pragma unroll
-						for (int e = 0; e < 4; e++)
-						{
-							const int dof = 32 * tile + 16 * h + 4 * e + (lane >> 4);
-							if (dof < dofs) out[dof] = c.acc[h][p][e];
-						}
+					units &= units - 1;
+					const int jn = units ? __builtin_ctzll(units) : j;
+					typename C::S sn;
+					c.load(sn, node(jn), DP);
+					__builtin_amdgcn_sched_barrier(0);
+					c.begin(node(j));
+					c.contract(sb, basis + (size_t)(f0 * kUnits + j) * U * kWave, __builtin_amdgcn_readlane(av, j), lane);
+					if (!units) break;
+					sb = sn;
+					j = jn;
 				}
 			}
 		}
-		if (a.stats && lane == 0)
+		c.finish();
+
+		// the parts' sums, in order, through LDS (the basis is done with)
+		double* const buf = lds + (size_t)(tile - a.dt_base) * C::kAcc * kWave + lane;
+		for (int p = 0; p + 1 < parts; p++)
 		{
-			if (tile == a.dt_base)
+			__syncthreads();
+			if (part == p)
 			{
-				atomicAdd(&a.stats[0], (unsigned long long)st_nodes);
-				atomicAdd(&a.stats[2], (unsigned long long)st_chunks);
-				atomicAdd(&a.stats[3], 1ull);
+#pragma unroll
+				for (int r = 0; r < C::kAcc; r++) buf[r * kWave] = p ? buf[r * kWave] + c.get(r) : c.get(r);
 			}
-			atomicAdd(&a.stats[4], (unsigned long long)st_mfma);
+		}
+		if (a.stats && threadIdx.x == 0) atomicAdd(&a.stats[3], 1ull);
+		__syncthreads();
+		if (part == parts - 1)
+		{
+			const bool split = nseg > 1;
+			double* const part_s = a.partial + ldc(&pl->partial_base) + (seg * count + blk * kWave) * DP;
+#pragma unroll
+			for (int i0 = 0; i0 < C::kAcc; i0 += 4)
+			{
+				const int qp = C::point(i0, lane);
+				const uint32_t oq = (uint32_t)__shfl((int)orig, qp, 64);
+				double* out = split ? part_s + (int64_t)qp * DP : a.y + (int64_t)oq * a.ldy;
+#pragma unroll
+				for (int i = i0; i < i0 + 4; i++)
+				{
+					const double v = parts > 1 ? buf[i * kWave] + c.get(i) : c.get(i);
+					const int dof = 32 * tile + C::dof(i, lane);
+					if (qp < np && dof < dofs) out[dof] = v;
+				}
+			}
 		}
 	}
 }
 
 size_t sweep_direct_lds_bytes(int dim, int hats_max)
 {
-	return (size_t)dim * kWave * 8 + (size_t)hats_max * 8 + 16;
+	return (size_t)kDW * kBasisBytes + (size_t)dim * kWave * 8 + (size_t)hats_max * 8 + 8 + 4 * kDW;
 }
 
 const void* sweep_direct_kernel_ptr(int prec)
 {
-	switch (prec)
-	{
-	case HDDM_LB_FP64: return (const void*)&sweep_direct_kernel<HDDM_LB_FP64>;
-	case HDDM_LB_F16X2: return (const void*)&sweep_direct_kernel<HDDM_LB_F16X2>;
-	case HDDM_LB_BF16X3: return (const void*)&sweep_direct_kernel<HDDM_LB_BF16X3>;
-	case HDDM_LB_F32: return (const void*)&sweep_direct_kernel<HDDM_LB_F32>;
-	}
+	if (prec == HDDM_LB_FP64) return (const void*)&sweep_direct_kernel<HDDM_LB_FP64>;
+	if (prec == HDDM_LB_F32) return (const void*)&sweep_direct_kernel<HDDM_LB_F32>;
 	return nullptr;
 }
 
