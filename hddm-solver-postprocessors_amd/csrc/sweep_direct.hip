@@ -35,8 +35,10 @@
 //
 // Measured (ms; walking sweeps -> every wave forming the basis of its own tile
 // -> here): D=59 / 281,077 nodes / 128 dofs / 16,384 points F32 32.5 -> 19.7 ->
-// 16.0, FP64 82.3 -> 27.8 -> 21.8. At D=59 some 70 % of the nodes meet a point
-// of any block; the MFMAs of those are 5.3 ms of the F32 time.
+// 15.5, FP64 82.3 -> 27.8 -> 21.7. At D=59 85 % of the nodes meet a point of
+// any block; their MFMAs are 6.4 ms of the F32 time, forming the basis 3.1, the
+// folds 1.0; 40 % of the wave cycles wait (barriers of the rounds, LDS, surplus
+// rows; with three or four units' rows on their way 15.8 and more).
 #include "sweep_common.h"
 #include "kernels.h"
 
@@ -48,6 +50,7 @@ namespace {
 
 constexpr int kDW = kDirectWaves;
 constexpr int kBasisBytes = 8192;               // per wave
+constexpr int kAhead = 2;                       // units whose surplus rows are on their way
 
 typedef double dv4_t __attribute__((ext_vector_type(4)));
 typedef float fv32_t __attribute__((ext_vector_type(32)));
@@ -510,29 +513,39 @@ __global__ void __launch_bounds__(64 * kDW) __attribute__((amdgpu_waves_per_eu(2
 				else __builtin_amdgcn_wave_barrier();
 				if (!on) continue;
 				// The units of this wave's share, in node order; while one is
-				// contracted the next one's surplus rows load.
+				// contracted the surplus rows of the next ones load.
 				const uint32_t av = lane < (f1 - f0) * kUnits ? alive[f0 * kUnits + lane] : 0u;
 				uint64_t units = __builtin_amdgcn_ballot_w64(av != 0u);
 				if (!units) continue;
 				const int wfirst = s0 + f0 + (tb + i) * kDW;
-				int j = __builtin_ctzll(units);
 				auto node = [&](int u) { return (wfirst + u / kUnits) * kWin + sub * C::kSub + (u % kUnits) * U; };
-				typename C::S sb;
-				c.load(sb, node(j), DP);
-#pragma unroll 1
-				for (;;)
-				{
+				// (past the last unit its rows load again: with no branch around
+				// the loads, a wait can leave the later ones on their way)
+				typename C::S sb[kAhead];
+				int j[kAhead], at = 0;
+				uint32_t um[kAhead];
+				auto next = [&](int k) {
+					at = units ? __builtin_ctzll(units) : at;
+					um[k] = units ? __builtin_amdgcn_readlane(av, at) : 0u;
 					units &= units - 1;
-					const int jn = units ? __builtin_ctzll(units) : j;
-					typename C::S sn;
-					c.load(sn, node(jn), DP);
-					__builtin_amdgcn_sched_barrier(0);
-					c.begin(node(j));
-					c.contract(sb, basis + (size_t)(f0 * kUnits + j) * U * kWave, __builtin_amdgcn_readlane(av, j), lane);
-					if (!units) break;
-					sb = sn;
-					j = jn;
-				}
+					j[k] = at;
+					c.load(sb[k], node(at), DP);
+				};
+#pragma unroll
+				for (int k = 0; k < kAhead; k++) next(k);
+#pragma unroll 1
+				do
+				{
+#pragma unroll
+					for (int k = 0; k < kAhead; k++)
+					{
+						c.begin(node(j[k]));
+						c.contract(sb[k], basis + (size_t)(f0 * kUnits + j[k]) * U * kWave, um[k], lane);
+						__builtin_amdgcn_sched_barrier(0);
+						next(k);
+						__builtin_amdgcn_sched_barrier(0);
+					}
+				} while (um[0]);
 			}
 		}
 		c.finish();
