@@ -775,14 +775,21 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 	const int ns = ctx->tables_n;
 	const int bb = bucket_bits(npoints, ns, ctx->opt_sort);
 	const int64_t nb = (int64_t)(ns + 1) << bb;
-	HIP_TRY(launch_fill_u32(sc.hist, nb, 0u, st));
-	HIP_TRY(launch_bucket_key(npoints, x, ldx, sid, ctx->d_state_ok, ns, ctx->dim, bb, sc.bkey, sc.hist, st));
 	const bool walking = cfg.kind == TuneConfig::kWalking, table = cfg.kind == TuneConfig::kTable;
 	const int nt = walking ? 0 : split_waves(cfg.kind, prec);
 	const int groups = walking ? 1 : split_groups(ctx, nt, npoints);
-	HIP_TRY(launch_scan_plan(sc.hist, sc.cursor, nb, bb, ns, ctx->d_states, ctx->d_cost_order,
-		sc.plans, sc.hdr, walking && !cfg.ws && cfg.walk == kWalkLds ? cfg.waves : 1, 0, nt, groups, st));
-	HIP_TRY(launch_scatter(npoints, sc.bkey, sc.cursor, sc.perm, st));
+	const int group = walking && !cfg.ws && cfg.walk == kWalkLds ? cfg.waves : 1;
+	if (npoints <= kSmallPoints && nb <= kSmallBuckets)
+		HIP_TRY(launch_small_plan(npoints, x, ldx, sid, ctx->d_state_ok, ns, ctx->dim, nb, bb, ctx->d_states, ctx->d_cost_order,
+			sc.plans, sc.hdr, sc.perm, group, nt, groups, st));
+	else
+	{
+		HIP_TRY(launch_fill_u32(sc.hist, nb, 0u, st));
+		HIP_TRY(launch_bucket_key(npoints, x, ldx, sid, ctx->d_state_ok, ns, ctx->dim, bb, sc.bkey, sc.hist, st));
+		HIP_TRY(launch_scan_plan(sc.hist, sc.cursor, nb, bb, ns, ctx->d_states, ctx->d_cost_order,
+			sc.plans, sc.hdr, group, 0, nt, groups, st));
+		HIP_TRY(launch_scatter(npoints, sc.bkey, sc.cursor, sc.perm, st));
+	}
 
 	const void* kern = table ? sweep_table_kernel_ptr(sweep_prec(prec)) : !walking ? sweep_direct_kernel_ptr(sweep_prec(prec))
 		: cfg.ws ? sweep_ws_kernel_ptr(prec, xbanks_for(ctx->dim), ctx->fmax_all, cfg.nc)

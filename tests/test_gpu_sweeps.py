@@ -122,3 +122,31 @@ def test_adjoint_node_subsets(case):
     print("  errors", err, flush=True)
     assert err[0] <= 1e-10 and err[1] <= 1e-12
     assert np.array_equal(dx0, dxr)
+
+
+@pytest.mark.parametrize("npts", [1, 63, 1023, 1025, 2047, 2048, 2049])
+@pytest.mark.parametrize("sort", [0, 1])
+def test_point_order_and_plan_of_small_batches(npts, sort):
+    """Both sides of the size up to which one workgroup orders the points and
+    plans the items: three states, rows of an unknown state untouched."""
+    dim, dofs = 6, 8
+    r = np.random.default_rng(npts)
+    c = hddm_lb.Context(0)
+    c.set_option(hddm_lb.OPT_SORT_POINTS, sort)
+    states = []
+    for s in range(3):
+        ii, jj, lv, ix = hddm_lb.generate_grid(dim, 2, 4, 0.5, 11 + s, 300)
+        S = r.standard_normal((ii.shape[0], dofs))
+        c.upload_state(s, ii, jj, S)
+        states.append((ii, jj, S))
+    X = hddm_lb.synthetic_points(npts, dim, 5)
+    sid = r.integers(0, 4, npts).astype(np.int32)
+    print("points", npts, "sort", sort, flush=True)
+    y = run_forward(c, X, sid, hddm_lb.FP64)
+    c.close()
+    assert np.isnan(y[sid == 3]).all()
+    for s, (ii, jj, S) in enumerate(states):
+        at = sid == s
+        if at.any():
+            den = oracle.forward(ii, jj, np.ones((len(S), 1)), X[at]).max() * np.abs(S).max()
+            assert np.abs(y[at] - oracle.forward(ii, jj, S, X[at])).max() <= 1e-12 * den
