@@ -29,9 +29,9 @@
 //
 // Measured against the per-tile kernels (ms, before -> here, 32 dofs): D=20 /
 // 100,005 nodes / 65,536 points (37.7 million alive nodes of blocks) dx 16.6 ->
-// 7.2, dS 14.4 -> 7.3 (4.9 without its atomics); D=16 / 60,010 nodes / 100,003
-// points dx 8.7 -> 5.0, dS 9.9 -> 4.9; D=8 / 3,937 nodes / 16 dofs / 20,000
-// points both 1.64 -> 0.31.
+// 7.0, dS 14.4 -> 7.3 (4.9 without its atomics); D=16 / 60,010 nodes / 100,003
+// points dx 8.7 -> 4.9, dS 9.9 -> 4.9; D=8 / 3,937 nodes / 16 dofs / 20,000
+// points both 1.64 -> 0.30.
 #include "sweep_common.h"
 #include "hat_table.h"
 #include "kernels.h"
@@ -278,6 +278,8 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 #pragma unroll
 						for (int h = 0; h < 2; h++)
 						{
+							// no second eight: rows 8 .. repeat the first, not added
+							if (h && slots - j0 <= 8) continue;
 							uint32_t r[8];
 							double f[8], b[8];
 #pragma unroll
@@ -354,35 +356,48 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 							v[4 * e + 2] = b2;
 							v[4 * e + 3] = b3;
 						}
+						// The second eight only where there are some: half of the
+						// windows' last batches have none.
 						uint32_t r[16];
 						double f[16];
+						auto form = [&](int h) {
 #pragma unroll
-						for (int k = 0; k < 16; k++) r[k] = __builtin_amdgcn_readlane(rv, j0 + k);
+							for (int k = 8 * h; k < 8 * h + 8; k++) r[k] = __builtin_amdgcn_readlane(rv, j0 + k);
 #pragma unroll
-						for (int k = 0; k < 16; k++) f[k] = *(const double*)((const char*)lds + ((r[k] & rowmask) | lane8));
+							for (int k = 8 * h; k < 8 * h + 8; k++) f[k] = *(const double*)((const char*)lds + ((r[k] & rowmask) | lane8));
 #pragma unroll
-						for (int k = 0; k < 16; k += 4)
-						{
-							double b[4];
-							Path<224>::mulp4(P, r + k, f + k, b);
+							for (int k = 8 * h; k < 8 * h + 8; k += 4)
+							{
+								double b[4];
+								Path<224>::mulp4(P, r + k, f + k, b);
 #pragma unroll
-							for (int m = 0; m < 4; m++) v[k + m] *= b[m];
-						}
-						// empty slots: the product may be that of an infinity and zero
-						if (slots - j0 < 16)
-						{
+								for (int m = 0; m < 4; m++) v[k + m] *= b[m];
+							}
+							// empty slots: the product may be that of an infinity and zero
+							if (slots - j0 < 8 * h + 8)
+							{
 #pragma unroll
-							for (int k = 1; k < 16; k++) v[k] = k < slots - j0 ? v[k] : 0.0;
-						}
+								for (int k = 8 * h + 1; k < 8 * h + 8; k++) v[k] = k < slots - j0 ? v[k] : 0.0;
+							}
+						};
 						// The edges, from the last slot back: an edge's nodes come
 						// before it. The edges above the first slot get this batch's
 						// part of their sums.
+						auto edges = [&](int h) {
 #pragma unroll
-						for (int k = 15; k >= 0; k--)
+							for (int k = 8 * h + 7; k >= 8 * h; k--)
+							{
+								const uint32_t inf = __builtin_amdgcn_readlane(iv, j0 + k);
+								edge_done<XB>(dx0, dx1, R, inf, r[k], v[k], hat_slope(f[k], inf));
+							}
+						};
+						form(0);
+						if (slots - j0 > 8)
 						{
-							const uint32_t inf = __builtin_amdgcn_readlane(iv, j0 + k);
-							edge_done<XB>(dx0, dx1, R, inf, r[k], v[k], hat_slope(f[k], inf));
+							form(1);
+							edges(1);
 						}
+						edges(0);
 						const uint32_t upinf = info[up / (8u * kWave)];
 #pragma unroll 1
 						for (int t = depth - 1; t >= 0; t--)
