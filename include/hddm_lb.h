@@ -49,8 +49,8 @@ typedef struct hddm_lb_grid hddm_lb_grid;
 
 /* arithmetic of the contraction (the basis is always formed in FP64) */
 #define HDDM_LB_FP64    0  /* FP64 VALU contraction, FP64 accumulation */
-#define HDDM_LB_F16X2   1  /* MFMA f16: basis hi+lo x scaled surplus hi+lo, 3 products */
-#define HDDM_LB_BF16X3  2  /* MFMA bf16: 3-term splits, 6 products */
+#define HDDM_LB_F16X2   1  /* MFMA f16: basis hi+lo x scaled surplus hi+lo, 3 products; F32 where that is faster */
+#define HDDM_LB_BF16X3  2  /* MFMA bf16: 3-term splits, 6 products; F32 where that is faster */
 #define HDDM_LB_F32     3  /* MFMA f32: basis f32 x surplus f32 */
 
 /* options for hddm_lb_set_option */
@@ -178,7 +178,8 @@ int hddm_lb_forward_host(hddm_lb_ctx* ctx, int64_t npoints,
  * wave-specialized kernel the products g.S and B^T g run on the bf16 MFMA
  * units with each F32 operand split into three bf16 parts (F32 accuracy),
  * F32 accumulation per 64-point chunk and FP64 accumulation beyond; the
- * per-tile kernels compute in FP64 for either precision). Stream-ordered. */
+ * hat-table and per-tile kernels compute in FP64 for either precision).
+ * Stream-ordered. */
 int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 	const double* x, int64_t ldx, const int32_t* state_ids,
 	const double* gbar, int64_t ldg, double* dx, int64_t lddx,
@@ -220,7 +221,10 @@ int hddm_lb_last_stats(hddm_lb_ctx* ctx, uint64_t* stats);
  * v_mfma_f32_32x32x16_{f16,bf16} on the split paths, v_mfma_f64_16x16x4f64
  * on the FP64 path of the wave-specialized sweep, 0 on the FP64 VALU path);
  * stats[5] is the number of (point, node) pairs with a non-zero basis value
- * that the contraction received (wave-specialized sweep only, else 0). */
+ * that the contraction received (wave-specialized sweep only, else 0).
+ * On the direct and hat-table sweeps: stats[0] the ops or nodes that a point
+ * of their block meets, [1] 0, [2] 32-node chunks (F32) or units of eight
+ * (FP64) with one, [4] v_mfma_f32_32x32x1_2b issued, 0 on FP64. */
 int hddm_lb_last_stats_n(hddm_lb_ctx* ctx, uint64_t* stats, int n);
 
 /* With HDDM_LB_OPT_STATS set, counters of the last wave-specialized adjoint,
