@@ -121,7 +121,7 @@ constexpr uint32_t kTabEmpty = 2u * (kTabMaxFactors - 1);
 // Waves of the hat-table sweep's workgroup (one workgroup per CU).
 constexpr int kTableWavesF32 = 12;
 constexpr int kTableWavesFP64 = 8;
-// Waves of the direct sweep's.
+// Waves of the direct sweep's workgroup.
 constexpr int kDirectWaves = 8;
 // Nodes per selection window of the direct sweep: one node per lane.
 constexpr int kWin = 64;

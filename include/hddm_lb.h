@@ -240,13 +240,13 @@ int hddm_lb_last_adjoint_stats(hddm_lb_ctx* ctx, uint64_t* stats, int n);
 int hddm_lb_host_call_stats(hddm_lb_ctx* ctx, int64_t* requests, int64_t* batches);
 
 /* Sweep configuration of the last hddm_lb_forward: config[0] formulation
- * (1 each wave walks and contracts, 2 wave-specialized), [1] waves per
+ * (1 one kind of wave, 2 wave-specialized), [1] waves per
  * workgroup, [2] dof tiles of 32 per launch, [3] keys the autotuner has
  * tuned on this context, [4] forwards it served from its cache. */
 int hddm_lb_last_config(hddm_lb_ctx* ctx, int* config);
 
-/* Configuration of the last hddm_lb_adjoint: config[0] kernels (1 per-tile,
- * 2 wave-specialized), [1] dS copies of owned units (0: dS added with
+/* Configuration of the last hddm_lb_adjoint: config[0] kernels (1 per-tile
+ * or hat-table, 2 wave-specialized), [1] dS copies of owned units (0: dS added with
  * atomics), [2] dS copies summed after the kernels (1: none), [3] most node
  * segments of a state in the kernels' tables. */
 int hddm_lb_last_adjoint_config(hddm_lb_ctx* ctx, int* config);
