@@ -153,7 +153,8 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 		__syncthreads();
 		// The hats at the block's points, and the points inside their
 		// supports. For dx a value carries the sign of u = x i - j, and 1.0
-		// is the peak alone: u > 0 that rounds to 1 is the value below it.
+		// is the peak alone (u is 0 of either sign: -0.0 at x = -0.0 and
+		// j = 0): u > 0 that rounds to 1 is the value below it.
 		{
 			const int hats = ldc(&sd->hats);
 			const u4_t* ht = (const u4_t*)ldc(&sd->hat);
@@ -171,7 +172,7 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 				const double u = (*(const double*)((const char*)X + lane * 8 + e[0]) + f64_from_high(e[2])) * f64_from_high(e[1]);
 				const double v = fmax(1.0 - fabs(u), 0.0);
 				const uint64_t in = __builtin_amdgcn_ballot_w64(v > 0.0) & valid;
-				lds[h * kWave + lane] = DS ? v : __builtin_copysign(v == 1.0 && u > 0.0 ? 1.0 - 0x1p-53 : v, u);
+				lds[h * kWave + lane] = DS ? v : u < 0.0 ? -v : v == 1.0 && u > 0.0 ? 1.0 - 0x1p-53 : v;
 				if (lane == 0)
 				{
 					M[h] = in;
