@@ -110,14 +110,15 @@ constexpr int kMaxHats = 2048;
 // Record of an op in the hat-table sweep: the row of its hat in LDS (512 bytes
 // a row), twice its depth, its node's place after the window's first. The
 // empty record is the row of zeros at the deepest depth, where no product is
-// a parent's. Stored xor the empty record (0 is empty).
+// a parent's, and ends no node: it takes the surplus row of zeros, where a
+// node's may be infinite or no number. Stored xor the empty record (0 is empty).
 constexpr uint32_t kTabRow = 0x3fe00u;
 constexpr uint32_t kTabDepth2 = 0xffu;    // alone in the low byte: GPR indexing reads that
 constexpr uint32_t kTabPrefix = 0x40000u; // the op ends no node: it has no surplus
 constexpr int kTabNodeShift = 20;
 constexpr int kMaxTableHats = 512;
 constexpr int kTabMaxFactors = 7;
-constexpr uint32_t kTabEmpty = 2u * (kTabMaxFactors - 1);
+constexpr uint32_t kTabEmpty = 2u * (kTabMaxFactors - 1) | kTabPrefix;
 // Waves of the hat-table sweep's workgroup (one workgroup per CU).
 constexpr int kTableWavesF32 = 12;
 constexpr int kTableWavesFP64 = 8;

@@ -228,8 +228,17 @@ struct Contract<HDDM_LB_FP64>
 		const double* row = basis + (lane >> 4) * kWave + (lane & 15);
 #pragma unroll
 		for (int q = 0; q < 2; q++)
-			if ((mask >> (4 * q)) & 15u)
+			if (const uint32_t qm = (mask >> (4 * q)) & 15u)
 			{
+				// dead nodes of the four: their basis is 0, and so is what stands
+				// for their surplus, which may be no number
+				double s0 = s.v[q][0], s1 = s.v[q][1];
+				if (qm != 15u)
+				{
+					const bool live = (qm >> (lane >> 4)) & 1u;
+					s0 = live ? s0 : 0.0;
+					s1 = live ? s1 : 0.0;
+				}
 				double b[4];
 #pragma unroll
 				for (int p = 0; p < 4; p++) b[p] = row[4 * q * kWave + 16 * p];
@@ -237,8 +246,8 @@ struct Contract<HDDM_LB_FP64>
 				for (int p = 0; p < 4; p++)
 					if (__builtin_amdgcn_ballot_w64(b[p] != 0.0))
 					{
-						acc[0][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(s.v[q][0], b[p], acc[0][p], 0, 0, 0);
-						acc[1][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(s.v[q][1], b[p], acc[1][p], 0, 0, 0);
+						acc[0][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(s0, b[p], acc[0][p], 0, 0, 0);
+						acc[1][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(s1, b[p], acc[1][p], 0, 0, 0);
 					}
 			}
 	}

@@ -45,3 +45,51 @@ def test_adjoint_at_negative_zero(dim, dofs):
     for dx in got:
         assert np.abs(dx - dxo).max() <= 1e-10 * np.abs(dxo).max()
     assert np.array_equal(got[0], got[1])
+
+
+# dim, base, depth, nodes of the grid (0: all), dofs: hat tables of one tile and
+# of two; more hats than those take, one tile and three
+GRIDS = [(6, 3, 4, 0, 20), (16, 2, 6, 6000, 40), (4, 7, 8, 0, 8), (59, 3, 4, 0, 65)]
+
+
+@pytest.mark.parametrize("npts", [1, 3, 200])
+@pytest.mark.parametrize("grid", GRIDS, ids=lambda g: "d%d-c%d" % (g[0], g[4]))
+def test_nodes_that_no_point_meets_do_not_count(grid, npts):
+    """Surpluses of nodes outside every point's block leave the results alone
+    whatever they are: infinite and NaN ones give the results of zeros, bit for
+    bit, forward and dx."""
+    import torch
+    dim, base, depth, nodes, dofs = grid
+    ii, jj, lv, ix = hddm_lb.generate_grid(dim, base, depth, 0.3 if nodes else 0.0, 7, nodes)
+    r = np.random.default_rng(npts)
+    if len(ii) > 8000:
+        rows = np.sort(r.choice(len(ii), 6000, replace=False))
+        ii, jj = np.ascontiguousarray(ii[rows]), np.ascontiguousarray(jj[rows])
+    # supports in the lower half of the first dimension
+    low = (ii[:, 0] > 0) & (jj[:, 0] + 1 <= ii[:, 0] // 2)
+    assert low.sum() > 5
+    S = r.standard_normal((len(ii), dofs))
+    X = hddm_lb.synthetic_points(npts, dim, 9)
+    X[:, 0] = 0.5 + 0.5 * X[:, 0]
+    G = r.standard_normal((npts, dofs))
+    x = torch.from_numpy(X).cuda()
+    c = hddm_lb.Context(0)
+    got = []
+    for bad in (0.0, np.inf, np.nan):
+        S[low] = bad
+        S[np.flatnonzero(low)[::2]] *= -1.0
+        c.upload_state(0, ii, jj, S)
+        res = []
+        for prec in (hddm_lb.FP64, hddm_lb.F32):
+            print("dim", dim, "points", npts, "surplus", bad, "precision", prec, flush=True)
+            y = torch.full((npts, dofs), np.nan, dtype=torch.float64, device="cuda")
+            c.forward(x, y, None, prec)
+            torch.cuda.synchronize()
+            res.append(y.cpu().numpy())
+        if dim <= 32 and dofs <= 32:
+            res.append(adjoint(c, X, G)[0])
+        got.append(res)
+    c.close()
+    for a in got:
+        for p, q in zip(a, got[0]):
+            assert np.isfinite(p).all() and np.array_equal(p, q)
