@@ -242,6 +242,7 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 				}
 				uint32_t iv = 0;   // infos by slot
 				if constexpr (!DS) iv = info[(rv & kTabRow) >> 9];
+				const uint64_t bare = __builtin_amdgcn_ballot_w64((rv & kTabPrefix) != 0u);   // slots without a surplus
 				// The hats above slot j, by depth in the lanes, as offsets of
 				// their rows; depth lanes count.
 				auto above = [&](int j, int& depth) -> uint32_t {
@@ -374,11 +375,12 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 #pragma unroll
 								for (int m = 0; m < 4; m++) v[k + m] *= b[m];
 							}
-							// empty slots: the product may be that of an infinity and zero
-							if (slots - j0 < 8 * h + 8)
+							// Empty slots and prefixes that are no nodes add nothing: an
+							// infinite gradient times their zeros is no number.
+							if ((bare >> (j0 + 8 * h)) & 0xffu)
 							{
 #pragma unroll
-								for (int k = 8 * h + 1; k < 8 * h + 8; k++) v[k] = k < slots - j0 ? v[k] : 0.0;
+								for (int k = 8 * h; k < 8 * h + 8; k++) v[k] = r[k] & kTabPrefix ? 0.0 : v[k];
 							}
 						};
 						// The edges, from the last slot back: an edge's nodes come

@@ -93,3 +93,29 @@ def test_nodes_that_no_point_meets_do_not_count(grid, npts):
     for a in got:
         for p, q in zip(a, got[0]):
             assert np.isfinite(p).all() and np.array_equal(p, q)
+
+
+def test_infinite_gradient_at_prefixes_that_are_no_nodes():
+    """A prefix that is no node has no surplus and adds nothing, also to the dx
+    of a point whose upstream gradient is infinite."""
+    r = np.random.default_rng(3)
+    dim, dofs = 8, 4
+    on = np.unique(r.random((200, dim)) < 0.4, axis=0)
+    # products of hats (2, 2), whose slope is +2 at every point below 1; those of
+    # even size only, so that every other prefix is none
+    on = on[on.sum(1) % 2 == 0]
+    on = on[(on.sum(1) >= 2) & (on.sum(1) <= 6)]
+    ii = np.where(on, 2, 0).astype(np.int32)
+    jj = ii.copy()
+    S = 1.0 + r.random((len(ii), dofs))
+    X = 0.6 + 0.3 * r.random((5, dim))
+    G = 1.0 + r.random((5, dofs))
+    G[2, 1] = np.inf
+    c = hddm_lb.Context(0)
+    c.upload_state(0, ii, jj, S)
+    dx, ds = adjoint(c, X, G)
+    c.close()
+    dxo = oracle.adjoint(ii, jj, S, X, G)[0]
+    assert np.array_equal(np.isinf(dxo[2]), on.any(0)) and np.array_equal(dx[2], dxo[2])
+    rest = [0, 1, 3, 4]
+    assert np.abs(dx[rest] - dxo[rest]).max() <= 1e-10 * np.abs(dxo[rest]).max()
