@@ -692,20 +692,22 @@ int split_segments(const hddm_lb_ctx* ctx, int nt, int g)
 	return most;
 }
 
-// Workgroups per 64-point block (the nodes are split between them).
+// Workgroups per 64-point block (the nodes are split between them). The same for
+// all batches of one block, whatever their size.
 int split_groups(const hddm_lb_ctx* ctx, int nt, int64_t npoints)
 {
 	const int64_t nblk = (npoints + kWave - 1) / kWave;
 	int64_t g = std::max<int64_t>(1, std::min<int64_t>(kSplitGroups / nblk, 256));
 	// partials: at most kSplitPartialBytes, or what the walking sweeps' segments take
-	const int64_t most = std::max<int64_t>(kSplitPartialBytes, npoints * ctx->max_nseg_dp * (int64_t)sizeof(double));
-	while (g > 1 && npoints * split_partial(ctx, nt, (int)g) * (int64_t)sizeof(double) > most) g--;
+	const int64_t pts = std::max<int64_t>(npoints, kWave);
+	const int64_t most = std::max<int64_t>(kSplitPartialBytes, pts * ctx->max_nseg_dp * (int64_t)sizeof(double));
+	while (g > 1 && pts * split_partial(ctx, nt, (int)g) * (int64_t)sizeof(double) > most) g--;
 	return (int)g;
 }
 
 // FP64 elements of the segment partials of a direct or hat-table sweep of any
-// precision.
-int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints)
+// precision, nodes shared out for split_points points (0: npoints).
+int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints, int64_t split_points)
 {
 	int64_t most = 0;
 	for (int prec : { HDDM_LB_FP64, HDDM_LB_F32 })
@@ -713,13 +715,13 @@ int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints)
 		const int kind = sweep_kind(ctx, prec);
 		if (kind == TuneConfig::kWalking) continue;
 		const int nt = split_waves(kind, prec);
-		most = std::max(most, npoints * split_partial(ctx, nt, split_groups(ctx, nt, npoints)));
+		most = std::max(most, npoints * split_partial(ctx, nt, split_groups(ctx, nt, split_points ? split_points : npoints)));
 	}
 	return most;
 }
 
 // Allocates scratch for npoints; must run outside graph capture.
-int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints)
+int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, int64_t split_points)
 {
 	int rc = prepare_tables(ctx);
 	if (rc) return rc;
@@ -733,7 +735,7 @@ int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints)
 	if ((rc = grow(sc.plans, sc.cap_plans, (size_t)ns))) return rc;
 	if ((rc = grow(sc.hdr, sc.cap_hdr, 1))) return rc;
 	// the tuner runs both kinds of sweep
-	size_t part = (size_t)split_partial_elems(ctx, npoints);
+	size_t part = (size_t)split_partial_elems(ctx, npoints, split_points);
 	if (sweep_kind(ctx, HDDM_LB_F16X2) == TuneConfig::kWalking || ctx->opt_autotune) part = std::max(part, (size_t)npoints * (size_t)ctx->max_nseg_dp);
 	if (part > 0)
 		if ((rc = grow(sc.partial, sc.cap_partial, part))) return rc;
@@ -777,7 +779,7 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 	const int64_t nb = (int64_t)(ns + 1) << bb;
 	const bool walking = cfg.kind == TuneConfig::kWalking, table = cfg.kind == TuneConfig::kTable;
 	const int nt = walking ? 0 : split_waves(cfg.kind, prec);
-	const int groups = walking ? 1 : split_groups(ctx, nt, npoints);
+	const int groups = walking ? 1 : split_groups(ctx, nt, cfg.split_points ? cfg.split_points : npoints);
 	const int group = walking && !cfg.ws && cfg.walk == kWalkLds ? cfg.waves : 1;
 	if (npoints <= kSmallPoints && nb <= kSmallBuckets)
 		HIP_TRY(launch_small_plan(npoints, x, ldx, sid, ctx->d_state_ok, ns, ctx->dim, nb, bb, ctx->d_states, ctx->d_cost_order,
@@ -865,18 +867,20 @@ int check_forward_args(hddm_lb_ctx* ctx, int64_t npoints, const double* x, int64
 
 } // namespace hddm_lb
 
-extern "C" int hddm_lb_forward(hddm_lb_ctx* ctx, int64_t npoints,
+// An eager forward; split_points as in TuneConfig.
+static int forward_eager(hddm_lb_ctx* ctx, int64_t npoints,
 	const double* x, int64_t ldx, const int32_t* state_ids,
-	double* y, int64_t ldy, int precision, void* stream)
+	double* y, int64_t ldy, int precision, void* stream, int64_t split_points)
 {
 	int rc = check_forward_args(ctx, npoints, x, ldx, y, ldy, precision);
 	if (rc) return rc;
 	if (npoints == 0) return HDDM_LB_SUCCESS;
 	DeviceGuard g(ctx->device);
 	hipStream_t st = (hipStream_t)stream;
-	if ((rc = prepare_scratch(ctx, ctx->scratch, npoints))) return rc;
+	if ((rc = prepare_scratch(ctx, ctx->scratch, npoints, split_points))) return rc;
 	if ((rc = scratch_wait(ctx, st))) return rc;
 	TuneConfig cfg = default_config(ctx, precision);
+	cfg.split_points = split_points;
 	if (ctx->opt_autotune && (rc = autotune(ctx, npoints, x, ldx, state_ids, y, ldy, precision, st, cfg)))
 		return rc;
 	ctx->last_timed = ctx->opt_timing;
@@ -884,6 +888,13 @@ extern "C" int hddm_lb_forward(hddm_lb_ctx* ctx, int64_t npoints,
 	rc = enqueue_forward(ctx, ctx->scratch, npoints, x, ldx, state_ids, y, ldy, precision, st, cfg, ctx->opt_timing);
 	if (rc) return rc;
 	return scratch_mark(ctx, st);
+}
+
+extern "C" int hddm_lb_forward(hddm_lb_ctx* ctx, int64_t npoints,
+	const double* x, int64_t ldx, const int32_t* state_ids,
+	double* y, int64_t ldy, int precision, void* stream)
+{
+	return forward_eager(ctx, npoints, x, ldx, state_ids, y, ldy, precision, stream, 0);
 }
 
 extern "C" int hddm_lb_last_stats_n(hddm_lb_ctx* ctx, uint64_t* stats, int n)
@@ -995,10 +1006,11 @@ struct hddm_lb_plan
 	}
 };
 
-// The staged forward of host buffers; the caller holds ctx->run_mu.
+// The staged forward of host buffers; the caller holds ctx->run_mu. split_points
+// as in TuneConfig.
 static int forward_host_run(hddm_lb_ctx* ctx, int64_t npoints,
 	const double* x, int64_t ldx, const int32_t* state_ids,
-	double* y, int64_t ldy, int precision)
+	double* y, int64_t ldy, int precision, int64_t split_points)
 {
 	int rc = HDDM_LB_SUCCESS;
 	DeviceGuard g(ctx->device);
@@ -1053,8 +1065,8 @@ static int forward_host_run(hddm_lb_ctx* ctx, int64_t npoints,
 	}
 	else
 	{
-		rc = hddm_lb_forward(ctx, npoints, ctx->d_xstage, ldx, state_ids ? ctx->d_sidstage : nullptr,
-			ctx->d_ystage, ldy, precision, st);
+		rc = forward_eager(ctx, npoints, ctx->d_xstage, ldx, state_ids ? ctx->d_sidstage : nullptr,
+			ctx->d_ystage, ldy, precision, st, split_points);
 		if (rc) return rc;
 	}
 	HIP_TRY(hipMemcpyAsync(ctx->h_ystage, ctx->d_ystage, sizeof(double) * npoints * ldy, hipMemcpyDeviceToHost, st));
@@ -1066,7 +1078,17 @@ static int forward_host_run(hddm_lb_ctx* ctx, int64_t npoints,
 // Requests taken into one coalesced batch, in points.
 constexpr int64_t kCoalesceMax = 4096;
 
-// Runs queued requests of one precision as one forward: rows packed with
+// Points of a coalesced batch: the partials of a batch that shares out nodes as
+// one block does fit their limit.
+static int64_t coalesce_max(const hddm_lb_ctx* ctx)
+{
+	const int64_t per = split_partial_elems(ctx, 1, kSmallBatch) * (int64_t)sizeof(double);
+	return per ? std::max<int64_t>(kSmallBatch, std::min<int64_t>(kCoalesceMax, kSplitPartialBytes / per)) : kCoalesceMax;
+}
+
+// Runs queued requests of one precision as one forward, which shares out nodes
+// as a block of the smallest size does: a request's results do not depend on
+// those that happen to be queued with it; rows packed with
 // ldx = dim and ldy = the widest state's dofs (the callers' y rows are packed
 // too, so columns and rows the forward leaves alone come back unchanged).
 static int run_coalesced(hddm_lb_ctx* ctx, const std::vector<HostRequest*>& batch)
@@ -1075,7 +1097,7 @@ static int run_coalesced(hddm_lb_ctx* ctx, const std::vector<HostRequest*>& batc
 	if (batch.size() == 1)
 	{
 		const HostRequest* r = batch[0];
-		return forward_host_run(ctx, r->n, r->x, r->ldx, r->sid, r->y, r->ldy, r->prec);
+		return forward_host_run(ctx, r->n, r->x, r->ldx, r->sid, r->y, r->ldy, r->prec, kSmallBatch);
 	}
 	int maxdofs = 0;
 	for (auto& s : ctx->states) if (s && s->loaded) maxdofs = std::max(maxdofs, s->desc.dofs);
@@ -1095,7 +1117,7 @@ static int run_coalesced(hddm_lb_ctx* ctx, const std::vector<HostRequest*>& batc
 			sid[(size_t)row] = r->sid ? r->sid[p] : 0;
 		}
 	}
-	const int rc = forward_host_run(ctx, tot, xs.data(), dim, sid.data(), ys.data(), maxdofs, batch[0]->prec);
+	const int rc = forward_host_run(ctx, tot, xs.data(), dim, sid.data(), ys.data(), maxdofs, batch[0]->prec, kSmallBatch);
 	if (rc) return rc;
 	row = 0;
 	for (const HostRequest* r : batch)
@@ -1117,10 +1139,10 @@ extern "C" int hddm_lb_forward_host(hddm_lb_ctx* ctx, int64_t npoints,
 	if (npoints > kSmallBatch || !ctx->opt_coalesce)
 	{
 		std::lock_guard<std::mutex> run(ctx->run_mu);
-		return forward_host_run(ctx, npoints, x, ldx, state_ids, y, ldy, precision);
+		return forward_host_run(ctx, npoints, x, ldx, state_ids, y, ldy, precision, npoints > kSmallBatch ? 0 : kSmallBatch);
 	}
 	// small call: queue it; whichever waiting thread finds no batch running
-	// takes every queued request of its precision (up to kCoalesceMax points)
+	// takes every queued request of its precision (up to coalesce_max points)
 	// and runs them as one forward
 	HostRequest me{ npoints, x, ldx, state_ids, y, ldy, precision, HDDM_LB_SUCCESS, false };
 	std::unique_lock<std::mutex> lk(ctx->comb_mu);
@@ -1130,10 +1152,11 @@ extern "C" int hddm_lb_forward_host(hddm_lb_ctx* ctx, int64_t npoints,
 		if (ctx->comb_busy) { ctx->comb_cv.wait(lk); continue; }
 		ctx->comb_busy = true;
 		std::vector<HostRequest*> batch;
+		const int64_t most = ctx->comb_queue.size() > 1 ? coalesce_max(ctx) : kCoalesceMax;
 		int64_t tot = 0;
 		for (auto it = ctx->comb_queue.begin(); it != ctx->comb_queue.end();)
 		{
-			if ((*it)->prec == precision && tot + (*it)->n <= kCoalesceMax)
+			if ((*it)->prec == precision && tot + (*it)->n <= most)
 			{
 				tot += (*it)->n;
 				batch.push_back(*it);

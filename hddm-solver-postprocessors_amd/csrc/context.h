@@ -96,6 +96,9 @@ struct TuneConfig
 	// the sweeps that select nodes by hat masks (sweep_direct.hip, sweep_table.hip)
 	enum Kind { kWalking = 0, kDirect = 1, kTable = 2 };
 	int kind = kWalking;
+	// Batch size that the direct and hat-table sweeps share out nodes for; 0: the
+	// call's. The order of a point's sums depends on it.
+	int64_t split_points = 0;
 };
 
 } // namespace hddm_lb
@@ -218,11 +221,11 @@ int noalloc_init(hddm_lb_ctx* ctx);
 int scratch_wait(hddm_lb_ctx* ctx, hipStream_t st);
 // Marks the end of an eager call's use of ctx->scratch on st.
 int scratch_mark(hddm_lb_ctx* ctx, hipStream_t st);
-int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints);
+int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, int64_t split_points = 0);
 int sweep_kind(const hddm_lb_ctx* ctx, int prec);
 int split_groups(const hddm_lb_ctx* ctx, int nt, int64_t npoints);
 int split_segments(const hddm_lb_ctx* ctx, int nt, int g);
-int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints);
+int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints, int64_t split_points = 0);
 // Workgroups that a direct or hat-table sweep aims at when it splits a small
 // batch's nodes. Measured (ms at 1, 2, 4, 8, 16 workgroups per 64-point block):
 // hat table, F32, D=20 / 100,005 nodes / 1,024 blocks 2.81, 2.79, 2.83, 3.02,

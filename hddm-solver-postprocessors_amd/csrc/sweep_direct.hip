@@ -31,7 +31,8 @@
 //         zero is skipped.
 // Groups of nodes, folds and which wave adds which are fixed by the layout,
 // and what is skipped is exactly zero, so a point's result does not depend on
-// the points it shares a block with.
+// the points it shares a block with (its last bits do on how many workgroups
+// share a block's nodes, see split_groups).
 //
 // Measured (ms; walking sweeps -> every wave forming the basis of its own tile
 // -> here): D=59 / 281,077 nodes / 128 dofs / 16,384 points F32 32.5 -> 19.7 ->

@@ -34,7 +34,8 @@
 //         layout by two rounds of row swaps; a 16-point column tile where all
 //         four are zero is skipped.
 // Skipped terms are exactly zero and folds are fixed by the layout, so a
-// point's result does not depend on the points it shares a block with.
+// point's result does not depend on the points it shares a block with (its last
+// bits do on how many workgroups share a block's nodes, see split_groups).
 //
 // Measured against the walking sweeps (ms, before -> here): D=16 / 60,010
 // nodes / 32 dofs / 2^20 points F32 15.7 -> 14.4 and 100,003 points F32 2.58

@@ -132,6 +132,11 @@ int hddm_lb_state_info(hddm_lb_ctx* ctx, int istate,
  *   x         [npoints x ldx] FP64 coordinates in [0, 1]
  *   state_ids [npoints] int32 state of each point, or NULL for state 0
  *   y         [npoints x ldy] FP64; row p receives dofs(state_ids[p]) values
+ * Repeating a call repeats its bits. A point's result does not depend on the
+ * other points, but the order of its sums depends on the batch size: small
+ * batches share out a state's nodes between workgroups. Batches of up to 64
+ * points all do so in the same way; results of batches of other sizes may
+ * differ in the last bits.
  * Stream-ordered on `stream` (a hipStream_t, NULL for the default stream). */
 int hddm_lb_forward(hddm_lb_ctx* ctx, int64_t npoints,
 	const double* x, int64_t ldx, const int32_t* state_ids,
@@ -157,7 +162,8 @@ int hddm_lb_forward_noalloc(hddm_lb_ctx* ctx, int64_t npoints,
  * x and y go through pinned staging buffers (one DMA each way); a call of at
  * most 64 points replays a captured forward (one graph launch), and calls of
  * at most 64 points made concurrently from several threads are queued and
- * run as one batched forward (HDDM_LB_OPT_COALESCE). */
+ * run as one batched forward (HDDM_LB_OPT_COALESCE), which gives each the bits
+ * of its call made alone. */
 int hddm_lb_forward_host(hddm_lb_ctx* ctx, int64_t npoints,
 	const double* x, int64_t ldx, const int32_t* state_ids,
 	double* y, int64_t ldy, int precision);

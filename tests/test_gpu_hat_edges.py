@@ -119,3 +119,81 @@ def test_infinite_gradient_at_prefixes_that_are_no_nodes():
     assert np.array_equal(np.isinf(dxo[2]), on.any(0)) and np.array_equal(dx[2], dxo[2])
     rest = [0, 1, 3, 4]
     assert np.abs(dx[rest] - dxo[rest]).max() <= 1e-10 * np.abs(dxo[rest]).max()
+
+
+def test_host_calls_do_not_depend_on_what_is_queued_with_them():
+    """Small host calls of several threads are run as one batch; each gives the
+    bits of the call made alone, however many were queued."""
+    import threading
+    dim, dofs, n, nthreads = 16, 12, 60, 16
+    ii, jj, lv, ix = hddm_lb.generate_grid(dim, 2, 7, 0.3, 7, 60000)
+    c = hddm_lb.Context(0)
+    c.upload_state(0, ii, jj, np.random.default_rng(1).standard_normal((len(ii), dofs)))
+    X = [hddm_lb.synthetic_points(n, dim, 20 + t) for t in range(nthreads)]
+    alone = [c.forward_host(x, np.zeros((n, dofs)), None, hddm_lb.FP64).copy() for x in X]
+    bad = []
+
+    def worker(t):
+        for k in range(20):
+            if not np.array_equal(c.forward_host(X[t], np.zeros((n, dofs)), None, hddm_lb.FP64), alone[t]):
+                bad.append((t, k))
+    before = c.host_call_stats()
+    th = [threading.Thread(target=worker, args=(t,)) for t in range(nthreads)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    after = c.host_call_stats()
+    print("requests", after[0] - before[0], "batches", after[1] - before[1], "different", len(bad), flush=True)
+    c.close()
+    assert not bad
+
+
+# dim, base, depth, probability, nodes of the grid (0: all), dofs: hat tables of
+# one tile and of four; direct, one tile and more than four
+BATCH_GRIDS = [(16, 2, 6, 0.3, 20000, 24), (24, 1, 6, 0.3, 12000, 128), (6, 6, 7, 0.0, 0, 8), (59, 2, 4, 0.0, 0, 150)]
+
+
+@pytest.mark.parametrize("grid", BATCH_GRIDS, ids=lambda g: "d%d-c%d" % (g[0], g[5]))
+def test_results_in_batches_of_other_sizes(grid):
+    """A point's forward has the same bits in every batch of up to 64 points,
+    and in one of the same size made as a plan or without allocations. Batches
+    of other sizes may share out a state's nodes in other runs: the same terms
+    in another order, to the tolerances of any order (1e-12 and 1e-6)."""
+    import torch
+    dim, base, depth, p, nodes, dofs = grid
+    r = np.random.default_rng(dim)
+    c = hddm_lb.Context(0)
+    for s, keep in enumerate((1.0, 0.4)):
+        ii, jj, lv, ix = hddm_lb.generate_grid(dim, base, depth, p, 7, nodes)
+        rows = np.flatnonzero(r.random(len(ii)) < keep)
+        c.upload_state(s, np.ascontiguousarray(ii[rows]), np.ascontiguousarray(jj[rows]), r.standard_normal((len(rows), dofs)))
+    big = 40000
+    x = torch.from_numpy(hddm_lb.synthetic_points(big, dim, 9)).cuda()
+    sid = torch.from_numpy(r.integers(0, 2, big).astype(np.int32)).cuda()
+
+    def run(n, prec):
+        y = torch.full((n, dofs), np.nan, dtype=torch.float64, device="cuda")
+        c.forward(x[:n], y, sid[:n], prec)
+        torch.cuda.synchronize()
+        return y
+    for prec in (hddm_lb.FP64, hddm_lb.F32):
+        ref, one = run(big, prec), run(64, prec)
+        for n in (1, 7, 64, 700, 3000, 13000):
+            print("dim", dim, "precision", prec, "points", n, flush=True)
+            a = run(n, prec)
+            if n <= 64:
+                assert torch.equal(a, one[:n])
+            assert (a - ref[:n]).abs().max() <= (1e-12 if prec == hddm_lb.FP64 else 1e-6) * ref.abs().max()
+            if n in (64, 3000):
+                b = torch.full_like(a, np.nan)
+                assert hddm_lb.lib.hddm_lb_forward_noalloc(c._h, n, x.data_ptr(), dim, sid.data_ptr(), b.data_ptr(), dofs,
+                                                           prec, torch.cuda.current_stream().cuda_stream) == 0
+                torch.cuda.synchronize()
+                d = torch.full_like(a, np.nan)
+                plan = c.plan(x[:n], d, sid[:n], prec)
+                plan.launch(torch.cuda.current_stream())
+                torch.cuda.synchronize()
+                assert torch.equal(b, a) and torch.equal(d, a)
+                del plan
+    c.close()
