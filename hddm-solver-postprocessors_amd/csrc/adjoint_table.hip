@@ -292,7 +292,7 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 							Path<224>::mulp4(P, r + 4, f + 4, b + 4);
 #pragma unroll
 							for (int k = 0; k < 8; k++) stage[k * kStageRow + lane] = b[k];
-							__builtin_amdgcn_wave_barrier();
+							wave_lds_order();
 							if (h == 0 || col >= 8)
 							{
 #pragma unroll
@@ -303,7 +303,7 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 									A[2 * m + 1] = v[1];
 								}
 							}
-							__builtin_amdgcn_wave_barrier();
+							wave_lds_order();
 						}
 						dv4_t acc[2] = { { 0.0, 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0, 0.0 } };
 #pragma unroll

@@ -23,6 +23,15 @@ __device__ __forceinline__ void lds_add(double* p, double v)
 		__HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// Between writes and reads of LDS that a wave's lanes exchange data through. The
+// wave's LDS operations complete in order, so no instruction is needed; the
+// compiler must keep that order.
+__device__ __forceinline__ void wave_lds_order()
+{
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+}
+
 // One work item: G neighbouring 64-point blocks of one state (one block per
 // wave of the workgroup) against one node segment of that state.
 struct ItemInfo

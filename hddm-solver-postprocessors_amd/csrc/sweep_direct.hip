@@ -452,7 +452,7 @@ __global__ void __launch_bounds__(64 * kDW) __attribute__((amdgpu_waves_per_eu(2
 				const int wn = (first + i * kDW) * kWin, n0 = wn + sub * C::kSub;
 				if (sub == 0) ahead = false;
 				if (tw > 1) __syncthreads();                // the round before has been contracted
-				else __builtin_amdgcn_wave_barrier();
+				else wave_lds_order();
 				if (lane < kUnits) alive[wave * kUnits + lane] = (uint8_t)(mask >> (8 * lane));
 				if (mask)
 				{
@@ -520,7 +520,7 @@ __global__ void __launch_bounds__(64 * kDW) __attribute__((amdgpu_waves_per_eu(2
 					}
 				}
 				if (tw > 1) __syncthreads();                // the round's basis is there
-				else __builtin_amdgcn_wave_barrier();
+				else wave_lds_order();
 				if (!on) continue;
 				// The units of this wave's share, in node order; while one is
 				// contracted the surplus rows of the next ones load.

@@ -107,7 +107,9 @@ struct TableContract<HDDM_LB_F32>
 
 	__device__ __forceinline__ void stage(S& s, const Rows& w, char* buf, int lane)
 	{
+		wave_lds_order();
 		*(f4v_t*)(buf + 16 * lane) = w.v;
+		wave_lds_order();
 #pragma unroll
 		for (int k = 0; k < 8; k++) s.v[k] = *(const float*)(buf + 128 * k + 4 * (lane & 31));
 	}
@@ -184,8 +186,10 @@ struct TableContract<HDDM_LB_FP64>
 
 	__device__ __forceinline__ void stage(S& s, const Rows& w, char* buf, int lane)
 	{
+		wave_lds_order();
 		*(d2v_t*)(buf + 16 * lane) = w.v[0];
 		*(d2v_t*)(buf + 1024 + 16 * lane) = w.v[1];
+		wave_lds_order();
 		const int k = lane >> 4;
 #pragma unroll
 		for (int q = 0; q < 2; q++)
