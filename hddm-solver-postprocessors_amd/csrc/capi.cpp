@@ -885,6 +885,7 @@ static int forward_eager(hddm_lb_ctx* ctx, int64_t npoints,
 		return rc;
 	ctx->last_timed = ctx->opt_timing;
 	ctx->last_cfg = cfg;
+	ctx->last_prec = precision;
 	rc = enqueue_forward(ctx, ctx->scratch, npoints, x, ldx, state_ids, y, ldy, precision, st, cfg, ctx->opt_timing);
 	if (rc) return rc;
 	return scratch_mark(ctx, st);
@@ -913,9 +914,9 @@ extern "C" int hddm_lb_last_config(hddm_lb_ctx* ctx, int* config)
 {
 	if (!ctx || !config) return set_error(HDDM_LB_ERROR_INVALID_VALUE, "last_config: NULL argument");
 	const TuneConfig& c = ctx->last_cfg;
-	const bool walking = c.kind == TuneConfig::kWalking, table = c.kind == TuneConfig::kTable;
+	const bool walking = c.kind == TuneConfig::kWalking;
 	config[0] = walking && c.ws ? 2 : 1;
-	config[1] = table ? kTableWavesF32 : !walking ? kDirectWaves : c.ws ? c.nc + 1 : c.waves;
+	config[1] = !walking ? split_waves(c.kind, ctx->last_prec) : c.ws ? c.nc + 1 : c.waves;
 	config[2] = !walking ? std::min(ctx->dt_needed, 4) : c.ws ? (c.nc == 4 ? 4 : 1) : c.slab;
 	config[3] = (int)ctx->tune_runs;
 	config[4] = (int)ctx->tune_hits;

@@ -207,6 +207,7 @@ struct hddm_lb_ctx
 	std::map<std::tuple<int, int, int64_t, int, int, int, int, int, int>, hddm_lb::TuneConfig> tuned;
 	int64_t tune_runs = 0, tune_hits = 0;   // keys tuned, forwards served from the cache
 	hddm_lb::TuneConfig last_cfg;           // configuration of the last eager forward
+	int last_prec = 0;                      // its precision
 	int last_adj[4] = { 0, 0, 0, 0 };       // hddm_lb_last_adjoint_config
 
 	~hddm_lb_ctx();

@@ -48,7 +48,7 @@ typedef struct hddm_lb_grid hddm_lb_grid;
 #define HDDM_LB_ERROR_UNSUPPORTED     8
 
 /* arithmetic of the contraction (the basis is always formed in FP64) */
-#define HDDM_LB_FP64    0  /* FP64 VALU contraction, FP64 accumulation */
+#define HDDM_LB_FP64    0  /* FP64 products, FP64 accumulation */
 #define HDDM_LB_F16X2   1  /* MFMA f16: basis hi+lo x scaled surplus hi+lo, 3 products; F32 where that is faster */
 #define HDDM_LB_BF16X3  2  /* MFMA bf16: 3-term splits, 6 products; F32 where that is faster */
 #define HDDM_LB_F32     3  /* MFMA f32: basis f32 x surplus f32 */
@@ -247,7 +247,8 @@ int hddm_lb_host_call_stats(hddm_lb_ctx* ctx, int64_t* requests, int64_t* batche
 
 /* Sweep configuration of the last hddm_lb_forward: config[0] formulation
  * (1 one kind of wave, 2 wave-specialized), [1] waves per
- * workgroup, [2] dof tiles of 32 per launch, [3] keys the autotuner has
+ * workgroup (hat-table sweep 12 in F32, 8 in FP64; direct 8; else at most 5),
+ * [2] dof tiles of 32 per launch, [3] keys the autotuner has
  * tuned on this context, [4] forwards it served from its cache. */
 int hddm_lb_last_config(hddm_lb_ctx* ctx, int* config);
 

@@ -197,3 +197,21 @@ def test_results_in_batches_of_other_sizes(grid):
                 assert torch.equal(b, a) and torch.equal(d, a)
                 del plan
     c.close()
+
+
+def test_last_config_gives_the_waves_of_the_kernel_that_ran():
+    import torch
+    # (grid, formulation) and the waves in FP64 and F32: hat tables, direct, walking
+    for (dim, base, depth, form), waves in (((6, 3, 4, 0), (8, 12)), ((4, 7, 8, 0), (8, 8)), ((6, 3, 4, 1), (4, 4))):
+        c = hddm_lb.Context(0)
+        ii, jj, lv, ix = hddm_lb.generate_grid(dim, base, depth, 0.0, 7, 0)
+        c.upload_state(0, ii, jj, np.ones((len(ii), 8)))
+        c.set_option(hddm_lb.OPT_FORMULATION, form)
+        x = torch.full((100, dim), 0.3, dtype=torch.float64, device="cuda")
+        y = torch.zeros((100, 8), dtype=torch.float64, device="cuda")
+        for prec, want in zip((hddm_lb.FP64, hddm_lb.F32), waves):
+            print("dim", dim, "formulation", form, "precision", prec, flush=True)
+            c.forward(x, y, None, prec)
+            torch.cuda.synchronize()
+            assert c.last_config()["waves"] == want
+        c.close()
