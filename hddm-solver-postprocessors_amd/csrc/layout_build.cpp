@@ -168,6 +168,8 @@ int build_layout(int dim, int nno, int dofs,
 			const auto& prev = seq[L.order[n - 1]];
 			while (s < (int)cur.size() && s < (int)prev.size() &&
 				!(cur[s] < prev[s]) && !(prev[s] < cur[s])) s++;
+			// a copy of the predecessor: a sibling of it, with an op of its own
+			if (s > 0 && s == (int)cur.size()) s--;
 		}
 		S[n] = s;
 		L.shared[n] = (uint8_t)s;

@@ -164,6 +164,8 @@ __global__ void shared_kernel(int nno, const Factor* fact, const int32_t* nf, co
 		const Factor* a = fact + (int64_t)k * kMaxFactors;
 		const Factor* b = fact + (int64_t)p * kMaxFactors;
 		while (s < f && s < fp && a[s].d == b[s].d && a[s].i == b[s].i && a[s].j == b[s].j) s++;
+		// a copy of the predecessor: a sibling of it, with an op of its own
+		if (s > 0 && s == f) s--;
 	}
 	F[n] = f;
 	S[n] = s;
