@@ -355,7 +355,8 @@ static int finish_upload(hddm_lb_ctx* ctx, int istate, int dim, std::unique_ptr<
 		if (p) slot->bufs.push_back(p);
 		return p;
 	};
-	if (int rc = build_direct_tables(slot->desc, slot->centre_exact, alloc)) return rc;
+	auto drop = [&](void* p) { slot->bufs.pop_back(); dev_free(p); };
+	if (int rc = build_direct_tables(slot->desc, slot->centre_exact, alloc, drop)) return rc;
 	slot->loaded = true;
 	if ((size_t)istate >= ctx->states.size()) ctx->states.resize(istate + 1);
 	ctx->states[istate] = std::move(slot);

@@ -8,6 +8,8 @@
 #include "kernels.h"
 #include "layout_build.h"
 
+#include <cstddef>
+
 namespace hddm_lb {
 
 namespace {
@@ -15,14 +17,22 @@ namespace {
 constexpr int kHashSlots = 8192;    // four times the most hats
 constexpr int kHashProbes = 512;
 
+// Needed while the tables are built.
 struct HatTable
 {
 	unsigned long long key[kHashSlots];   // 0: free
 	uint32_t id[kHashSlots];
-	int total;                            // hats found
-	int overflow;                         // a key found no slot
-	int wide;                             // a dof column's largest value is out of F32's range
 };
+
+// In the place of the records of the hats that are none (ids below kHatFirst).
+struct HatCount
+{
+	int total;                            // hat ids
+	int overflow;                         // a key found no slot, or there are more than kMaxHats
+	int wide;                             // a dof column's largest value is out of F32's range
+	int found;                            // keys inserted
+};
+static_assert(sizeof(HatCount) <= kHatFirst * 16, "fits");
 
 // i is a power of two: its exponent, the dim and the centre name the hat.
 __device__ __forceinline__ unsigned long long hat_key(const uint32_t* e)
@@ -37,22 +47,15 @@ __device__ __forceinline__ uint32_t hat_slot(unsigned long long key)
 	return (uint32_t)(key >> 40) & (kHashSlots - 1);
 }
 
-__global__ void direct_init_kernel(HatTable* t)
-{
-	for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < kHashSlots; s += gridDim.x * blockDim.x) t->key[s] = 0ull;
-	if (blockIdx.x == 0 && threadIdx.x == 0) { t->total = 0; t->overflow = 0; t->wide = 0; }
-}
-
-// Padding nodes: phi = max(0, 1 - |0 x - 2|) = 0.
-__global__ void rec_init_kernel(int nno, int npad, uint32_t* rec)
-{
-	const int n = nno + blockIdx.x * blockDim.x + threadIdx.x;
-	if (n < npad) { rec[2 * n] = 0u; rec[2 * n + 1] = 0xc0000000u; }
-}
-
-__global__ void rec_kernel(int nops, const Op* __restrict__ ops, uint32_t* __restrict__ rec)
+// The empty hash, the records of padding nodes (phi = max(0, 1 - |0 x - 2|) = 0)
+// and of the nodes. One thread per hash slot or op.
+__global__ void rec_kernel(HatTable* __restrict__ t, HatCount* __restrict__ cnt, int nno, int npad, int nops, const Op* __restrict__ ops,
+	uint32_t* __restrict__ rec)
 {
 	const int q = blockIdx.x * blockDim.x + threadIdx.x;
+	if (q < kHashSlots) t->key[q] = 0ull;
+	if (q == 0) *cnt = HatCount{ 0, 0, 0, 0 };
+	if (q < npad - nno) { rec[2 * (nno + q)] = 0u; rec[2 * (nno + q) + 1] = 0xc0000000u; }
 	if (q >= nops) return;
 	const Op op = ops[q];
 	if (!(op.ctrl & kOpLast)) return;
@@ -84,10 +87,11 @@ __global__ void special_kernel(int nno, int npad, uint32_t* __restrict__ rec)
 	if (any & (kRecPrefix | kRecRoot)) rec[2 * (8 * o)] |= kRecSpecial;
 }
 
-__global__ void hat_insert_kernel(int64_t nent, const uint32_t* __restrict__ ftab, HatTable* t)
+// A state with too many hats gets no tables: the count stops the search early.
+__global__ void hat_insert_kernel(int64_t nent, const uint32_t* __restrict__ ftab, HatTable* t, HatCount* cnt)
 {
 	const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (k >= nent) return;
+	if (k >= nent || __hip_atomic_load(&cnt->overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
 	const uint32_t* e = ftab + 4 * k;
 	if (!e[3]) return;
 	const unsigned long long key = hat_key(e);
@@ -99,21 +103,22 @@ __global__ void hat_insert_kernel(int64_t nent, const uint32_t* __restrict__ fta
 		if (old == 0ull)
 		{
 			old = atomicCAS(&t->key[s], 0ull, key);
+			if (old == 0ull && atomicAdd(&cnt->found, 1) >= kMaxHats - kHatFirst) cnt->overflow = 1;
 			if (old == 0ull || old == key) return;
 		}
 	}
-	t->overflow = 1;
+	cnt->overflow = 1;
 }
 
 // One workgroup of 1024 threads: ids in slot order, the hats' records, and
 // whether the columns' largest values (2^14 to 2^15 iscale) lie in 2^-100 .. 2^100.
-__global__ void __launch_bounds__(1024) hat_number_kernel(HatTable* t, uint32_t* __restrict__ hat, int DP, const double* __restrict__ iscale)
+__global__ void __launch_bounds__(1024) hat_number_kernel(HatTable* t, HatCount* cnt, uint32_t* __restrict__ hat, int DP, const double* __restrict__ iscale)
 {
 	__shared__ int wsum[16];
 	constexpr int kPer = kHashSlots / 1024;
 	const int tid = threadIdx.x, lane = tid & 63;
 	for (int c = tid; c < DP; c += 1024)
-		if (iscale[c] < 0x1p-114 || iscale[c] > 0x1p+85) t->wide = 1;
+		if (iscale[c] < 0x1p-114 || iscale[c] > 0x1p+85) cnt->wide = 1;
 	int mine = 0;
 	for (int k = 0; k < kPer; k++) mine += t->key[tid * kPer + k] != 0ull;
 	int x = mine;
@@ -147,14 +152,14 @@ __global__ void __launch_bounds__(1024) hat_number_kernel(HatTable* t, uint32_t*
 		}
 		id++;
 	}
-	if (tid == 0) t->total = kHatFirst + total;
+	if (tid == 0) cnt->total = kHatFirst + total;
 }
 
 __global__ void hat_lookup_kernel(int nno, int npad, int fstride, int hstride, const uint32_t* __restrict__ ftab, const HatTable* __restrict__ t,
-	uint16_t* __restrict__ hid)
+	const HatCount* __restrict__ cnt, uint16_t* __restrict__ hid)
 {
 	const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (k >= (int64_t)npad * hstride) return;
+	if (k >= (int64_t)npad * hstride || cnt->overflow) return;
 	const int64_t n = k / hstride;
 	uint32_t id = n < nno ? kHatAll : kHatNone;
 	if (id == kHatAll)
@@ -204,7 +209,7 @@ int grid_for(int64_t n) { return (int)((n + 255) / 256); }
 
 // States with an index_i that is no power of two, or with more than kMaxHats
 // hats, get no tables (hats = 0).
-int build_direct_tables(StateDesc& d, bool centre_exact, const DeviceAlloc& alloc)
+int build_direct_tables(StateDesc& d, bool centre_exact, const DeviceAlloc& alloc, const DeviceDrop& drop)
 {
 	d.hats = 0;
 	if (!centre_exact) return HDDM_LB_SUCCESS;
@@ -212,48 +217,57 @@ int build_direct_tables(StateDesc& d, bool centre_exact, const DeviceAlloc& allo
 	const int fs = (int)d.fstride;
 	const int hs = d.max_depth > 8 ? 16 : (d.max_depth + 1) / 2 * 2;   // at most fstride
 	const int qpad = (d.nops + kWin - 1) / kWin * kWin;
-	// one allocation: it is small next to the layout, and each costs an upload
-	// of a few thousand nodes some 5 % (measured: six more, 0.66 -> 0.86 ms)
-	const size_t bytes[] = { (size_t)npad * 8, (size_t)npad * hs * sizeof(uint16_t), (size_t)qpad * sizeof(uint32_t),
-		(size_t)qpad * hs * sizeof(uint16_t), (size_t)(qpad / kWin) * sizeof(int32_t), (size_t)kMaxHats * 16, sizeof(HatTable) };
-	size_t off[8] = { 0 };
-	for (int k = 0; k < 7; k++) off[k + 1] = off[k] + (bytes[k] + 255) / 256 * 256;
+	// One allocation, small next to the layout (each costs an upload of a few
+	// thousand nodes some 5 %: measured with six more, 0.66 -> 0.86 ms). The
+	// hat-table sweep's records of a small state take the hash's place.
+	auto place = [](const size_t* bytes, int n, size_t* off) {
+		off[0] = 0;
+		for (int k = 0; k < n; k++) off[k + 1] = off[k] + (bytes[k] + 255) / 256 * 256;
+	};
+	const size_t bytes[] = { (size_t)npad * 8, (size_t)npad * hs * sizeof(uint16_t), (size_t)kMaxHats * 16, sizeof(HatTable) };
+	const size_t tbytes[] = { (size_t)qpad * sizeof(uint32_t), (size_t)qpad * hs * sizeof(uint16_t), (size_t)(qpad / kWin) * sizeof(int32_t) };
+	size_t off[5], toff[4];
+	place(bytes, 4, off);
+	place(tbytes, 3, toff);
 	int rc = HDDM_LB_SUCCESS;
-	char* const base = (char*)alloc(off[7], rc);
+	char* const base = (char*)alloc(off[4], rc);
 	if (rc) return rc;
 	uint32_t* rec = (uint32_t*)(base + off[0]);
 	uint16_t* hid = (uint16_t*)(base + off[1]);
-	uint32_t* trec = (uint32_t*)(base + off[2]);
-	uint16_t* thid = (uint16_t*)(base + off[3]);
-	int32_t* tnode = (int32_t*)(base + off[4]);
-	uint32_t* hat = (uint32_t*)(base + off[5]);
-	HatTable* t = (HatTable*)(base + off[6]);
+	uint32_t* hat = (uint32_t*)(base + off[2]);
+	HatCount* cnt = (HatCount*)hat;
+	HatTable* t = (HatTable*)(base + off[3]);
 	const hipStream_t st = nullptr;
 	const int64_t nent = (int64_t)d.nno * fs;
-	hipLaunchKernelGGL(direct_init_kernel, dim3(8), dim3(256), 0, st, t);
-	hipLaunchKernelGGL(rec_init_kernel, dim3(1), dim3(64), 0, st, d.nno, npad, rec);
-	hipLaunchKernelGGL(rec_kernel, dim3(grid_for(d.nops)), dim3(256), 0, st, d.nops, d.ops, rec);
+	hipLaunchKernelGGL(rec_kernel, dim3(grid_for(d.nops > kHashSlots ? d.nops : kHashSlots)), dim3(256), 0, st, t, cnt, d.nno, npad,
+		d.nops, d.ops, rec);
+	hipLaunchKernelGGL(hat_insert_kernel, dim3(grid_for(nent)), dim3(256), 0, st, nent, d.ftab, t, cnt);
 	hipLaunchKernelGGL(prefix_kernel, dim3(grid_for((int64_t)d.nops * kWave)), dim3(256), 0, st, d.nno, d.nops, d.ops, rec);
 	hipLaunchKernelGGL(special_kernel, dim3(grid_for(npad / 8)), dim3(256), 0, st, d.nno, npad, rec);
-	hipLaunchKernelGGL(hat_insert_kernel, dim3(grid_for(nent)), dim3(256), 0, st, nent, d.ftab, t);
-	hipLaunchKernelGGL(hat_number_kernel, dim3(1), dim3(1024), 0, st, t, hat, d.dofs_pad, d.iscale);
+	hipLaunchKernelGGL(hat_number_kernel, dim3(1), dim3(1024), 0, st, t, cnt, hat, d.dofs_pad, d.iscale);
 	hipLaunchKernelGGL(hat_lookup_kernel, dim3(grid_for((int64_t)npad * hs)), dim3(256), 0, st, d.nno, npad, fs, hs, d.ftab,
-		(const HatTable*)t, hid);
-	hipLaunchKernelGGL(table_rec_kernel, dim3(grid_for(qpad)), dim3(256), 0, st, d.nops, qpad, hs, d.ops, (const uint16_t*)hid, trec,
-		thid, tnode);
+		(const HatTable*)t, (const HatCount*)cnt, hid);
 	HIP_TRY(hipGetLastError());
-	int found[3] = { 0, 0, 0 };
-	HIP_TRY(hipMemcpy(found, &t->total, sizeof(found), hipMemcpyDeviceToHost));
-	if (found[1] || found[0] > kMaxHats) return HDDM_LB_SUCCESS;
+	HatCount found = { 0, 0, 0, 0 };
+	HIP_TRY(hipMemcpy(&found, cnt, sizeof(found), hipMemcpyDeviceToHost));
+	if (found.overflow || found.total > kMaxHats) { drop(base); return HDDM_LB_SUCCESS; }
+	if (found.total <= kMaxTableHats && d.max_depth <= kTabMaxFactors)
+	{
+		char* const tb = toff[3] <= sizeof(HatTable) ? (char*)t : (char*)alloc(toff[3], rc);
+		if (rc) return rc;
+		d.trec = (uint32_t*)(tb + toff[0]);
+		d.thid = (uint16_t*)(tb + toff[1]);
+		d.tnode = (int32_t*)(tb + toff[2]);
+		hipLaunchKernelGGL(table_rec_kernel, dim3(grid_for(qpad)), dim3(256), 0, st, d.nops, qpad, hs, d.ops, (const uint16_t*)hid,
+			(uint32_t*)d.trec, (uint16_t*)d.thid, (int32_t*)d.tnode);
+		HIP_TRY(hipGetLastError());
+	}
 	d.rec = rec;
-	d.trec = trec;
-	d.thid = thid;
-	d.tnode = tnode;
 	d.hid = hid;
 	d.hat = hat;
 	d.hstride = hs;
-	d.f32_range = !found[2];
-	d.hats = found[0];
+	d.f32_range = !found.wide;
+	d.hats = found.total;
 	return HDDM_LB_SUCCESS;
 }
 

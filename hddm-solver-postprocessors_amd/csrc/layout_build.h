@@ -61,9 +61,12 @@ struct DeviceLayout
 // Device memory for the arrays of a DeviceLayout, owned by the caller; on
 // failure it sets rc and returns NULL.
 typedef std::function<void*(size_t, int&)> DeviceAlloc;
-// The direct sweep's tables of a state whose layout is built (d.ops, d.ftab);
-// d.hats stays 0 for a state the sweep does not take.
-int build_direct_tables(StateDesc& d, bool centre_exact, const DeviceAlloc& alloc);
+// Gives back the last allocation.
+typedef std::function<void(void*)> DeviceDrop;
+// The tables of the sweeps over hat masks, of a state whose layout is built
+// (d.ops, d.ftab); d.hats stays 0 for a state those do not take, d.trec null for
+// one that only the direct sweep takes.
+int build_direct_tables(StateDesc& d, bool centre_exact, const DeviceAlloc& alloc, const DeviceDrop& drop);
 // Returned by build_layout_device for inputs it leaves to build_layout
 // (out-of-range indices, more than 15 factors, too many nodes or ops), which
 // either builds them or reports the error.

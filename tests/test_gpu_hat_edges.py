@@ -215,3 +215,38 @@ def test_last_config_gives_the_waves_of_the_kernel_that_ran():
             torch.cuda.synchronize()
             assert c.last_config()["waves"] == want
         c.close()
+
+
+@pytest.mark.parametrize("hats,waves", [(510, 8), (511, 8), (2046, 8), (2047, 4), (12000, 4)])
+def test_number_of_hats(hats, waves):
+    """Up to 2,046 distinct hats a state runs on the sweeps over hat masks, past
+    that on the walking ones, also where the table that lists them is full."""
+    dim, dofs = 60, 9
+    every = [(d, 2 ** k, j) for k in range(1, 10) for d in range(dim) for j in range(0 if k == 1 else 1, 2 ** k + (k == 1), 1 if k == 1 else 2)]
+    every = [(d, i, j) for d, i, j in every if not (i == 2 and j == 1)]
+    r = np.random.default_rng(hats)
+    pick = every[:hats]
+    assert len(set(pick)) == hats
+    # the root, a node of one factor each, and pairs of them
+    ii, jj = np.zeros((1 + hats + 300, dim), np.int32), np.zeros((1 + hats + 300, dim), np.int32)
+    for n, (d, i, j) in enumerate(pick):
+        ii[1 + n, d], jj[1 + n, d] = i, j
+    for n in range(300):
+        for d, i, j in (pick[k] for k in r.choice(hats, 2, replace=False)):
+            ii[1 + hats + n, d], jj[1 + hats + n, d] = i, j
+    S = r.standard_normal((len(ii), dofs))
+    X = hddm_lb.synthetic_points(150, dim, 9)
+    import torch
+    c = hddm_lb.Context(0)
+    c.upload_state(0, ii, jj, S)
+    x = torch.from_numpy(X).cuda()
+    y = torch.full((150, dofs), np.nan, dtype=torch.float64, device="cuda")
+    print("hats", hats, flush=True)
+    c.forward(x, y, None, hddm_lb.FP64)
+    torch.cuda.synchronize()
+    got = c.last_config()["waves"]
+    c.close()
+    yo = oracle.forward(ii, jj, S, X)
+    den = oracle.forward(ii, jj, np.ones((len(ii), 1)), X).max() * np.abs(S).max()
+    assert got == waves
+    assert np.abs(y.cpu().numpy() - yo).max() <= 1e-12 * den
