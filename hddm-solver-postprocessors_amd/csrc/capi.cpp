@@ -780,7 +780,9 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 	const int64_t nb = (int64_t)(ns + 1) << bb;
 	const bool walking = cfg.kind == TuneConfig::kWalking, table = cfg.kind == TuneConfig::kTable;
 	const int nt = walking ? 0 : split_waves(cfg.kind, prec);
-	const int groups = walking ? 1 : split_groups(ctx, nt, cfg.split_points ? cfg.split_points : npoints);
+	int groups = walking ? 1 : split_groups(ctx, nt, cfg.split_points ? cfg.split_points : npoints);
+	// (the scratch was made for the same split: not reached)
+	if (groups > 1 && (size_t)npoints * (size_t)split_partial(ctx, nt, groups) > sc.cap_partial) groups = 1;
 	const int group = walking && !cfg.ws && cfg.walk == kWalkLds ? cfg.waves : 1;
 	if (npoints <= kSmallPoints && nb <= kSmallBuckets)
 		HIP_TRY(launch_small_plan(npoints, x, ldx, sid, ctx->d_state_ok, ns, ctx->dim, nb, bb, ctx->d_states, ctx->d_cost_order,
@@ -884,6 +886,7 @@ static int forward_eager(hddm_lb_ctx* ctx, int64_t npoints,
 	cfg.split_points = split_points;
 	if (ctx->opt_autotune && (rc = autotune(ctx, npoints, x, ldx, state_ids, y, ldy, precision, st, cfg)))
 		return rc;
+	cfg.split_points = split_points;   // the tuner's cache holds another call's
 	ctx->last_timed = ctx->opt_timing;
 	ctx->last_cfg = cfg;
 	ctx->last_prec = precision;
@@ -1206,6 +1209,7 @@ extern "C" int hddm_lb_plan_create(hddm_lb_ctx* ctx, int64_t npoints,
 	{
 		if ((rc = scratch_wait(ctx, (hipStream_t)stream))) return rc;
 		if ((rc = autotune(ctx, npoints, x, ldx, state_ids, y, ldy, precision, (hipStream_t)stream, cfg))) return rc;
+		cfg.split_points = 0;
 		if ((rc = scratch_mark(ctx, (hipStream_t)stream))) return rc;
 	}
 	std::unique_ptr<hddm_lb_plan> plan(new hddm_lb_plan);

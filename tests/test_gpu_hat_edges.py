@@ -250,3 +250,38 @@ def test_number_of_hats(hats, waves):
     den = oracle.forward(ii, jj, np.ones((len(ii), 1)), X).max() * np.abs(S).max()
     assert got == waves
     assert np.abs(y.cpu().numpy() - yo).max() <= 1e-12 * den
+
+
+def test_tuned_forward_after_coalesced_calls():
+    """The tuner's choice for a size is used by calls of that size however they
+    share out nodes: a batch of queued host calls, then device batches."""
+    import threading
+    import torch
+    dim, dofs, n = 16, 12, 64
+    ii, jj, lv, ix = hddm_lb.generate_grid(dim, 2, 7, 0.3, 7, 60000)
+    S = np.random.default_rng(1).standard_normal((len(ii), dofs))
+    c = hddm_lb.Context(0)
+    c.set_option(hddm_lb.OPT_AUTOTUNE, 1)
+    c.upload_state(0, ii, jj, S)
+    X = hddm_lb.synthetic_points(16 * n, dim, 20)
+    yo = oracle.forward(ii, jj, S, X)
+    out = np.zeros((16 * n, dofs))
+
+    def worker(t):
+        for k in range(5):
+            out[t * n:(t + 1) * n] = c.forward_host(X[t * n:(t + 1) * n], np.zeros((n, dofs)), None, hddm_lb.FP64)
+    th = [threading.Thread(target=worker, args=(t,)) for t in range(16)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    print("coalesced", flush=True)
+    assert np.abs(out - yo).max() <= 1e-12 * np.abs(yo).max()
+    for m in (1024, 512, 900):
+        x = torch.from_numpy(X[:m]).cuda()
+        y = torch.zeros((m, dofs), dtype=torch.float64, device="cuda")
+        print("points", m, flush=True)
+        c.forward(x, y, None, hddm_lb.FP64)
+        torch.cuda.synchronize()
+        assert np.abs(y.cpu().numpy() - yo[:m]).max() <= 1e-12 * np.abs(yo).max()
+    c.close()
