@@ -576,13 +576,15 @@ static int grow_dspart(Scratch& scr, size_t need)
 }
 
 // Whether the adjoint of one-tile states at D <= 32 takes the kernels over hat
-// tables: no option asks for the per-tile ones, and the tables fit.
-static bool adjoint_table_ok(const hddm_lb_ctx* ctx)
+// tables: no option asks for the per-tile ones, the tables fit, and the blocks
+// meet enough nodes.
+static bool adjoint_table_ok(const hddm_lb_ctx* ctx, int64_t npoints)
 {
 	return sweep_kind(ctx, HDDM_LB_FP64) != TuneConfig::kWalking && ctx->dt_needed == 1 && ctx->dim <= 32
 		&& ctx->hats_max <= kMaxTableHats && ctx->fmax_all <= kTabMaxFactors
 		&& adjoint_table_lds_bytes(true, ctx->dim, ctx->hats_max) <= ctx->max_lds
-		&& adjoint_table_lds_bytes(false, ctx->dim, ctx->hats_max) <= ctx->max_lds;
+		&& adjoint_table_lds_bytes(false, ctx->dim, ctx->hats_max) <= ctx->max_lds
+		&& !adjoint_walks(ctx, npoints);
 }
 
 extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
@@ -655,11 +657,11 @@ extern "C" int hddm_lb_adjoint(hddm_lb_ctx* ctx, int64_t npoints,
 	}
 	// the wave-specialized kernel splits states into finer node segments
 	const StateDesc* tables = ws ? ctx->d_states_adj : ctx->d_states;
-	// One dof tile, D <= 32: the kernels over hat tables where those exist. They
-	// were the faster ones at every size measured (dx and dS, ms, per-tile / hat
+	// One dof tile, D <= 32: the kernels over hat tables where those exist, apart
+	// from many blocks in one to three dimensions (dx and dS, ms, per-tile / hat
 	// table): D=20 / 100k / 32 dofs 31.0 / 14.3, D=16 / 60k / 32 dofs / 100,003
 	// points 18.7 / 9.7, D=8 / 3,937 nodes / 16 dofs / 20,000 points 1.64 / 0.30.
-	const bool table = !ws && adjoint_table_ok(ctx);
+	const bool table = !ws && adjoint_table_ok(ctx, npoints);
 	const int groups = table ? split_groups(ctx, adjoint_table_waves(), std::max<int64_t>(npoints, 1)) : 1;
 	const int max_nseg = table ? split_segments(ctx, adjoint_table_waves(), groups) : ws ? ctx->max_nseg_adj : ctx->max_nseg;
 

@@ -35,13 +35,16 @@ int autotune(hddm_lb_ctx* ctx, int64_t npoints, const double* x, int64_t ldx, co
 		if (s && s->loaded) { nodes += s->desc.nno; maxdofs = std::max(maxdofs, s->desc.dofs); }
 	int lg = 0;
 	while (((int64_t)1 << (lg + 1)) <= npoints) lg++;
+	const int kind = sweep_kind(ctx, prec);
 	auto key = std::make_tuple(prec, ctx->dim, nodes, maxdofs, lg, ctx->opt_form, ctx->opt_waves, ctx->opt_slab,
-		(int)cfg.kind);
+		kind);
 	auto hit = ctx->tuned.find(key);
 	if (hit != ctx->tuned.end()) { cfg = hit->second; ctx->tune_hits++; return HDDM_LB_SUCCESS; }
 
 	std::vector<TuneConfig> cands;
-	if (cfg.kind != TuneConfig::kWalking) cands.push_back(cfg);
+	cfg.kind = kind;
+	cfg.f32 = 0;
+	if (kind != TuneConfig::kWalking) cands.push_back(cfg);
 	cfg.kind = TuneConfig::kWalking;
 	if (ctx->opt_form != 2)
 		for (int waves : { 2, 4 })

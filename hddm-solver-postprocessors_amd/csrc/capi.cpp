@@ -235,6 +235,35 @@ extern "C" int hddm_lb_set_option(hddm_lb_ctx* ctx, int option, int64_t value)
 
 static int finish_upload(hddm_lb_ctx* ctx, int istate, int dim, std::unique_ptr<StateSlot> slot);
 
+// StateSlot::alive and visited from 256 nodes spread over the state: a hat of
+// width 2 / i meets a block of side s with probability 2 / i + s.
+static void estimate_alive(StateSlot& slot, int dim, int nno, const int32_t* index_i, int64_t ld_index)
+{
+	const int n = std::min(nno, 256);
+	float side[kSides], alive[kSides] = { 0 }, visited[kSides] = { 0 };
+	for (int k = 0; k < kSides; k++) side[k] = std::exp2(-0.5f * (float)k);
+	for (int j = 0; j < n; j++)
+	{
+		const int32_t* i = index_i + (int64_t)j * nno / n * ld_index;
+		float width[kWalkDims];
+		int f = 0;
+		for (int d = 0; d < dim; d++)
+			if (i[d] > 0) width[f++] = 2.0f / (float)i[d];
+		for (int k = 0; k < kSides; k++)
+		{
+			float p = 1.0f, before = 1.0f;
+			for (int t = 0; t < f; t++) { before = p; p *= std::min(1.0f, width[t] + side[k]); }
+			alive[k] += p;
+			visited[k] += before;
+		}
+	}
+	for (int k = 0; k < kSides; k++)
+	{
+		slot.alive[k] = alive[k] * (float)nno / (float)n;
+		slot.visited[k] = visited[k] * (float)nno / (float)n;
+	}
+}
+
 extern "C" int hddm_lb_upload_state(hddm_lb_ctx* ctx, int istate, int dim, int nno, int dofs,
 	const int32_t* index_i, const int32_t* index_j, int64_t ld_index,
 	const double* surplus, int64_t ld_surplus)
@@ -262,6 +291,7 @@ extern "C" int hddm_lb_upload_state(hddm_lb_ctx* ctx, int istate, int dim, int n
 				const int32_t i = index_i[k * ld_index + t], j = index_j[k * ld_index + t];
 				if ((i || j) && !(i > 0 && (i & (i - 1)) == 0)) { slot->centre_exact = false; break; }
 			}
+	if (index_i && index_j && ld_index >= dim && nno > 0 && dim <= kWalkDims) estimate_alive(*slot, dim, nno, index_i, ld_index);
 	std::memset(&d, 0, sizeof(d));
 	d.dim = dim; d.nno = nno; d.dofs = dofs;
 	d.nseg = 1;
@@ -662,6 +692,79 @@ int sweep_kind(const hddm_lb_ctx* ctx, int prec)
 	return ctx->table_ok ? TuneConfig::kTable : TuneConfig::kDirect;
 }
 
+// An estimate of StateSlot at a state's nblk blocks.
+static double at_blocks(const float* v, double nblk, int dim)
+{
+	const double at = std::min(std::max(2.0 * std::log2(nblk) / dim, 0.0), kSides - 1.0);
+	const int k = std::min((int)at, kSides - 2);
+	return v[k] + (at - k) * (v[k + 1] - v[k]);
+}
+
+static int loaded_states(const hddm_lb_ctx* ctx)
+{
+	int n = 0;
+	for (auto& s : ctx->states) n += s && s->loaded;
+	return n;
+}
+
+// Whether the per-tile adjoint beats the one over hat tables: many blocks that
+// meet next to no nodes (dx and dS, us, per-tile / hat table: 2^20 points D=1 /
+// 129 nodes 961 / 1,565, D=2 / 65 894 / 1,415, D=3 / 441 1,653 / 1,752, D=4 /
+// 1,105 2,918 / 2,548; 262,144 points D=2 387 / 436, D=3 641 / 528).
+bool adjoint_walks(const hddm_lb_ctx* ctx, int64_t npoints)
+{
+	if (ctx->dim > kWalkDims || npoints < 4096 * kWave) return false;
+	const double nblk = (double)npoints / kWave / loaded_states(ctx);
+	double most = 0.0;
+	for (auto& s : ctx->states)
+		if (s && s->loaded) most = std::max(most, at_blocks(s->visited, nblk, ctx->dim));
+	return most < nblk / 80;
+}
+
+// Whether the walking sweep beats the one over hat masks: blocks of a large batch
+// in few dimensions are small and meet few of a state's nodes. The walk leaves
+// out whole subtrees then, and its thousands of independent waves hide what a
+// workgroup per block waits for (points, hats, part sums: some 10 to 20 us a
+// block). Both times (us) from a model fitted to 906 forwards, D = 1 to 16, 65 to
+// 60,010 nodes, 8 to 128 dofs, 4,096 to 2^20 points. Measured (us, hat masks / walk, 8 dofs): 2^20
+// points D=4 / 7,537 nodes FP64 5,236 / 2,069, D=8 / 2,004 F32 1,736 / 1,090,
+// D=16 / 60,010 F32 14,374 / 15,391; 65,536 points D=6 / 44,689 FP64 1,763 /
+// 1,143, D=8 / 15,713 F32 363 / 1,182. The walk is taken where the model has it
+// ahead by an eighth. It runs split precisions in F32, as the others do.
+static bool walk_is_faster(const hddm_lb_ctx* ctx, int kind, int prec, int64_t npoints)
+{
+	if (ctx->dim > kWalkDims || npoints < 512 * kWave) return false;
+	const bool fp64 = prec == HDDM_LB_FP64, table = kind == TuneConfig::kTable;
+	const double nblk = (double)npoints / kWave / loaded_states(ctx);
+	// a visited op, blocks that keep the walk's waves busy, a block's fixed costs;
+	// a block's fixed costs, a hat, a node, a node that it meets
+	const double op = (fp64 ? 0.15 : 0.09) * (1.0 + (fp64 ? 0.55 : 1.8) / ctx->dim), busy = fp64 ? 6500 : 4900, walk_block = fp64 ? 3.8 : 3.9;
+	const double block = table ? (fp64 ? 8.5 : 12.0) : (fp64 ? 15.0 : 14.0), hat = table ? (fp64 ? 0.015 : 0.017) : 0.03;
+	const double node = table ? (fp64 ? 0.0024 : 0.0018) : (fp64 ? 0.0061 : 0.0036), met = table ? (fp64 ? 0.0036 : 0.0024) : (fp64 ? 0.0085 : 0.0066);
+	double chain = 40.0, rate = 0.0, walk = 40.0 + 2.1e-4 * (double)npoints, mask = walk;
+	for (auto& s : ctx->states)
+	{
+		if (!s || !s->loaded) continue;
+		const StateDesc& d = s->desc;
+		const int tiles = d.dofs_pad / 32, rest = tiles & 3;
+		const double visited = at_blocks(s->visited, nblk, ctx->dim), alive = at_blocks(s->alive, nblk, ctx->dim);
+		// the direct sweep forms a basis once for up to four tiles
+		const double passes = table ? tiles : tiles / 4 * 2.4 + std::min(rest, 2) + 0.2 * std::max(0, rest - 2);
+		chain = std::max(chain, tiles * visited * op / d.nseg);
+		rate += tiles * visited * op * nblk / busy;
+		walk += tiles * walk_block * nblk / 256;
+		mask += nblk / 256 * (block + hat * d.hats + (node * d.nno + met * alive) * passes);
+	}
+	return walk + std::sqrt(chain * chain + rate * rate) < 0.88 * mask;
+}
+
+// The sweep of a forward of npoints points.
+int forward_kind(const hddm_lb_ctx* ctx, int prec, int64_t npoints)
+{
+	const int kind = sweep_kind(ctx, prec);
+	return kind != TuneConfig::kWalking && walk_is_faster(ctx, kind, prec, npoints) ? TuneConfig::kWalking : kind;
+}
+
 // The precision that the direct and hat-table sweeps compute in.
 static int sweep_prec(int prec) { return prec == HDDM_LB_FP64 ? HDDM_LB_FP64 : HDDM_LB_F32; }
 
@@ -737,13 +840,15 @@ int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, int64_t spli
 	if ((rc = grow(sc.hdr, sc.cap_hdr, 1))) return rc;
 	// the tuner runs both kinds of sweep
 	size_t part = (size_t)split_partial_elems(ctx, npoints, split_points);
-	if (sweep_kind(ctx, HDDM_LB_F16X2) == TuneConfig::kWalking || ctx->opt_autotune) part = std::max(part, (size_t)npoints * (size_t)ctx->max_nseg_dp);
+	bool walks = ctx->opt_autotune;
+	for (int prec : { HDDM_LB_FP64, HDDM_LB_F32, HDDM_LB_F16X2 }) walks = walks || forward_kind(ctx, prec, npoints) == TuneConfig::kWalking;
+	if (walks) part = std::max(part, (size_t)npoints * (size_t)ctx->max_nseg_dp);
 	if (part > 0)
 		if ((rc = grow(sc.partial, sc.cap_partial, part))) return rc;
 	return HDDM_LB_SUCCESS;
 }
 
-TuneConfig default_config(hddm_lb_ctx* ctx, int prec)
+TuneConfig default_config(hddm_lb_ctx* ctx, int prec, int64_t npoints)
 {
 	TuneConfig c;
 	c.waves = ctx->opt_waves ? ctx->opt_waves : 4;
@@ -764,7 +869,8 @@ TuneConfig default_config(hddm_lb_ctx* ctx, int prec)
 	c.ws = ctx->opt_form == 2
 		|| (ctx->opt_form == 0 && prec == HDDM_LB_FP64 && xbanks_for(ctx->dim) == 4 && ctx->dt_needed >= 2);
 	c.nc = ctx->dt_needed >= 2 ? 4 : 2;
-	c.kind = sweep_kind(ctx, prec);
+	c.kind = forward_kind(ctx, prec, npoints);
+	c.f32 = c.kind != sweep_kind(ctx, prec) && prec != HDDM_LB_FP64;
 	return c;
 }
 
@@ -779,6 +885,7 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 	const int bb = bucket_bits(npoints, ns, ctx->opt_sort);
 	const int64_t nb = (int64_t)(ns + 1) << bb;
 	const bool walking = cfg.kind == TuneConfig::kWalking, table = cfg.kind == TuneConfig::kTable;
+	const int walk_prec = cfg.f32 ? HDDM_LB_F32 : prec;
 	const int nt = walking ? 0 : split_waves(cfg.kind, prec);
 	int groups = walking ? 1 : split_groups(ctx, nt, cfg.split_points ? cfg.split_points : npoints);
 	// (the scratch was made for the same split: not reached)
@@ -798,12 +905,12 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 
 	const void* kern = table ? sweep_table_kernel_ptr(sweep_prec(prec)) : !walking ? sweep_direct_kernel_ptr(sweep_prec(prec))
 		: cfg.ws ? sweep_ws_kernel_ptr(prec, xbanks_for(ctx->dim), ctx->fmax_all, cfg.nc)
-		: sweep_kernel_ptr(prec, cfg.slab, xbanks_for(ctx->dim), ctx->fmax_all, cfg.walk);
+		: sweep_kernel_ptr(walk_prec, cfg.slab, xbanks_for(ctx->dim), ctx->fmax_all, cfg.walk);
 	if (!kern) return set_error(HDDM_LB_ERROR_INVALID_VALUE, "forward: no sweep kernel for precision %d, dim %d", prec, ctx->dim);
 	const int waves = !walking ? nt : cfg.ws ? cfg.nc + 1 : cfg.waves;
 	const size_t lds = table ? sweep_table_lds_bytes(ctx->dim, ctx->hats_max, ctx->dt_needed)
 		: !walking ? sweep_direct_lds_bytes(ctx->dim, ctx->hats_max)
-		: cfg.ws ? sweep_ws_lds_bytes(prec, ctx->fmax_all) : sweep_lds_bytes(prec, cfg.waves, ctx->fmax_all, cfg.walk);
+		: cfg.ws ? sweep_ws_lds_bytes(prec, ctx->fmax_all) : sweep_lds_bytes(walk_prec, cfg.waves, ctx->fmax_all, cfg.walk);
 	HIP_TRY(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 	int per_cu = 0;
 	HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, waves * kWave, lds));
@@ -882,7 +989,7 @@ static int forward_eager(hddm_lb_ctx* ctx, int64_t npoints,
 	hipStream_t st = (hipStream_t)stream;
 	if ((rc = prepare_scratch(ctx, ctx->scratch, npoints, split_points))) return rc;
 	if ((rc = scratch_wait(ctx, st))) return rc;
-	TuneConfig cfg = default_config(ctx, precision);
+	TuneConfig cfg = default_config(ctx, precision, npoints);
 	cfg.split_points = split_points;
 	if (ctx->opt_autotune && (rc = autotune(ctx, npoints, x, ldx, state_ids, y, ldy, precision, st, cfg)))
 		return rc;
@@ -1204,7 +1311,7 @@ extern "C" int hddm_lb_plan_create(hddm_lb_ctx* ctx, int64_t npoints,
 	if (npoints < 1) return set_error(HDDM_LB_ERROR_INVALID_VALUE, "plan_create: npoints must be >= 1");
 	DeviceGuard g(ctx->device);
 	if ((rc = prepare_scratch(ctx, ctx->scratch, npoints))) return rc;
-	TuneConfig cfg = default_config(ctx, precision);
+	TuneConfig cfg = default_config(ctx, precision, npoints);
 	if (ctx->opt_autotune)
 	{
 		if ((rc = scratch_wait(ctx, (hipStream_t)stream))) return rc;

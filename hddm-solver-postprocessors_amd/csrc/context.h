@@ -26,6 +26,11 @@ struct DeviceGuard
 	~DeviceGuard();
 };
 
+// Sizes of blocks that a state's alive nodes are estimated for, and the most
+// dimensions in which a large batch's blocks are small enough to leave some out.
+constexpr int kSides = 17;
+constexpr int kWalkDims = 16;
+
 struct StateSlot
 {
 	bool loaded = false;
@@ -43,6 +48,9 @@ struct StateSlot
 	// node): the factor table's centre -j / i is then exact, which the
 	// wave-specialized adjoint's dx waves need
 	bool centre_exact = true;
+	// Estimates for blocks of side 2^(-k / 2): nodes that a block meets, and nodes
+	// whose prefix without the last factor does (D <= kWalkDims)
+	float alive[kSides] = { 0 }, visited[kSides] = { 0 };
 	~StateSlot();
 	void release();
 };
@@ -99,6 +107,7 @@ struct TuneConfig
 	// Batch size that the direct and hat-table sweeps share out nodes for; 0: the
 	// call's. The order of a point's sums depends on it.
 	int64_t split_points = 0;
+	int f32 = 0;       // a split precision on the walking sweeps is computed in F32
 };
 
 } // namespace hddm_lb
@@ -224,6 +233,8 @@ int scratch_wait(hddm_lb_ctx* ctx, hipStream_t st);
 int scratch_mark(hddm_lb_ctx* ctx, hipStream_t st);
 int prepare_scratch(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, int64_t split_points = 0);
 int sweep_kind(const hddm_lb_ctx* ctx, int prec);
+int forward_kind(const hddm_lb_ctx* ctx, int prec, int64_t npoints);
+bool adjoint_walks(const hddm_lb_ctx* ctx, int64_t npoints);
 int split_groups(const hddm_lb_ctx* ctx, int nt, int64_t npoints);
 int split_segments(const hddm_lb_ctx* ctx, int nt, int g);
 int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints, int64_t split_points = 0);
@@ -235,7 +246,7 @@ int64_t split_partial_elems(const hddm_lb_ctx* ctx, int64_t npoints, int64_t spl
 constexpr int64_t kSplitGroups = 1024;
 // Most segment partials that a split may cost.
 constexpr int64_t kSplitPartialBytes = (int64_t)32 << 20;
-TuneConfig default_config(hddm_lb_ctx* ctx, int prec);
+TuneConfig default_config(hddm_lb_ctx* ctx, int prec, int64_t npoints);
 int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double* x, int64_t ldx,
 	const int32_t* sid, double* y, int64_t ldy, int prec, hipStream_t st, const TuneConfig& cfg, bool timed);
 int autotune(hddm_lb_ctx* ctx, int64_t npoints, const double* x, int64_t ldx, const int32_t* sid,

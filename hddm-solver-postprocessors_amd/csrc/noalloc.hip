@@ -82,7 +82,9 @@ extern "C" int hddm_lb_forward_noalloc(hddm_lb_ctx* ctx, int64_t npoints,
 			(long long)npoints, off, kNoAllocScratchBytes);
 	// the direct and hat-table sweeps' partials are at most kSplitPartialBytes,
 	// and only for batches small enough to be split: they fit beside the rest
-	const size_t npart = sweep_kind(ctx, precision) != TuneConfig::kWalking ? (size_t)split_partial_elems(ctx, npoints)
+	// the default launch shape: tuning would create events and time candidates
+	const TuneConfig cfg = default_config(ctx, precision, npoints);
+	const size_t npart = cfg.kind != TuneConfig::kWalking ? (size_t)split_partial_elems(ctx, npoints)
 		: (size_t)npoints * (size_t)ctx->max_nseg_dp;
 	if (o_part + npart * sizeof(double) > kNoAllocScratchBytes)
 		return set_error(HDDM_LB_ERROR_INVALID_VALUE, "forward_noalloc: %zu bytes of partials do not fit the scratch array",
@@ -99,8 +101,6 @@ extern "C" int hddm_lb_forward_noalloc(hddm_lb_ctx* ctx, int64_t npoints,
 	sc.partial = npart > 0 ? (double*)(base + o_part) : nullptr;
 	sc.cap_partial = npart;
 	DeviceGuard g(ctx->device);
-	// the default launch shape: tuning would create events and time candidates
-	TuneConfig cfg = default_config(ctx, precision);
 	rc = enqueue_forward(ctx, sc, npoints, x, ldx, state_ids, y, ldy, precision, (hipStream_t)stream, cfg, false);
 	sc.bkey = sc.perm = sc.hist = sc.cursor = nullptr;
 	sc.plans = nullptr;

@@ -134,9 +134,9 @@ int hddm_lb_state_info(hddm_lb_ctx* ctx, int istate,
  *   y         [npoints x ldy] FP64; row p receives dofs(state_ids[p]) values
  * Repeating a call repeats its bits. A point's result does not depend on the
  * other points, but the order of its sums depends on the batch size: small
- * batches share out a state's nodes between workgroups. Batches of up to 64
- * points all do so in the same way; results of batches of other sizes may
- * differ in the last bits.
+ * batches share out a state's nodes between workgroups, and large ones in few
+ * dimensions may take another sweep. Batches of up to 64 points all do so in the
+ * same way; results of batches of other sizes may differ by rounding.
  * Stream-ordered on `stream` (a hipStream_t, NULL for the default stream). */
 int hddm_lb_forward(hddm_lb_ctx* ctx, int64_t npoints,
 	const double* x, int64_t ldx, const int32_t* state_ids,

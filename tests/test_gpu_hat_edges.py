@@ -285,3 +285,71 @@ def test_tuned_forward_after_coalesced_calls():
         torch.cuda.synchronize()
         assert np.abs(y.cpu().numpy() - yo[:m]).max() <= 1e-12 * np.abs(yo).max()
     c.close()
+
+
+# dim, base, depth, nodes of the grid (0: all), dofs, points of the large batch,
+# whether that walks; direct sweep and hat tables
+DENSE = [(4, 7, 8, 0, 8, 300000, True), (3, 6, 7, 0, 40, 1 << 20, True), (8, 1, 6, 2000, 8, 1 << 20, True),
+         (8, 1, 6, 2000, 8, 65536, False), (16, 2, 6, 6000, 40, 100000, False)]
+
+
+@pytest.mark.parametrize("grid", DENSE, ids=lambda g: "d%d-c%d-p%d" % (g[0], g[4], g[5]))
+def test_large_batches_in_few_dimensions(grid):
+    """Batches whose blocks meet few of a state's nodes run on the walking sweep;
+    its results are those of the other sweeps up to rounding (1e-12, 1e-6), for
+    every precision, with padded rows, two states and points of none."""
+    import torch
+    dim, base, depth, nodes, dofs, n, walks = grid
+    r = np.random.default_rng(dim)
+    c = hddm_lb.Context(0)
+    most = 0.0
+    for s, nd in enumerate((dofs, max(1, dofs // 2))):
+        ii, jj, lv, ix = hddm_lb.generate_grid(dim, base, depth, 0.3 if nodes else 0.0, 7, nodes)
+        S = r.standard_normal((len(ii), nd))
+        most = max(most, oracle.forward(ii, jj, np.ones((len(ii), 1)), r.random((500, dim))).max() * np.abs(S).max())
+        c.upload_state(s, ii, jj, S)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.rand((n, dim + 2), dtype=torch.float64, device="cuda", generator=g)
+    sid = torch.randint(-1, 3, (n,), dtype=torch.int32, device="cuda", generator=g)
+    for prec in (hddm_lb.FP64, hddm_lb.F32, hddm_lb.F16X2, hddm_lb.BF16X3):
+        y = torch.full((n, dofs + 3), 7.0, dtype=torch.float64, device="cuda")
+        c.forward(x[:, :dim], y[:, :dofs], sid, prec)
+        torch.cuda.synchronize()
+        print("dim", dim, "points", n, "precision", prec, c.last_config(), flush=True)
+        assert (c.last_config()["waves"] < 8) == walks
+        for p0 in range(0, n, n // 5):
+            m = min(3000, n - p0)
+            z = torch.full((m, dofs), 7.0, dtype=torch.float64, device="cuda")
+            c.forward(x[p0:p0 + m, :dim].contiguous(), z, sid[p0:p0 + m].contiguous(), prec)
+            torch.cuda.synchronize()
+            assert c.last_config()["waves"] >= 8
+            assert (y[p0:p0 + m, :dofs] - z).abs().max() <= (1e-12 if prec == hddm_lb.FP64 else 1e-6) * most
+        assert (y[:, dofs:] == 7.0).all() and (y[(sid < 0) | (sid > 1)] == 7.0).all()
+    c.close()
+
+
+@pytest.mark.parametrize("dim,n", [(1, 1 << 19), (2, 1 << 20), (4, 1 << 18)])
+def test_adjoint_of_large_batches_in_few_dimensions(dim, n):
+    """Both sides of the rule that leaves blocks that meet next to no nodes to the
+    per-tile kernels: dx and dS of the default are those of formulation 1."""
+    import torch
+    ii, jj, lv, ix = hddm_lb.generate_grid(dim, 5, 6, 0.0, 7, 0)
+    r = np.random.default_rng(dim)
+    S = r.standard_normal((len(ii), 6))
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.rand((n, dim), dtype=torch.float64, device="cuda", generator=g)
+    gb = torch.randn((n, 6), dtype=torch.float64, device="cuda", generator=g)
+    c = hddm_lb.Context(0)
+    c.upload_state(0, ii, jj, S)
+    got = []
+    for form in (0, 1):
+        c.set_option(hddm_lb.OPT_FORMULATION, form)
+        dx, ds = torch.full_like(x, np.nan), torch.full((S.size,), np.nan, dtype=torch.float64, device="cuda")
+        print("dim", dim, "points", n, "formulation", form, flush=True)
+        c.adjoint(x, gb, dx, ds)
+        torch.cuda.synchronize()
+        got.append((dx, ds))
+    c.close()
+    # dS sums n terms of size B g: 1e-12 of the largest leaves room for any order
+    for (a, b), tol in zip(zip(*got), (1e-10, 1e-12)):
+        assert (a - b).abs().max() <= tol * b.abs().max()
