@@ -677,10 +677,14 @@ int bucket_bits(int64_t npoints, int nstates, int sort)
 // LDS; the direct sweep otherwise.
 // The last two compute in FP64 or in F32. A split precision takes F32 there:
 // with the basis formed once for many nodes the F32 MFMAs cost less than
-// forming the split operands, and every product is exact to 24 bits instead
-// of 22. Measured (ms, walking / split operands in a direct sweep / F32):
-// F16X2 at D=24, 128 dofs, 30,011 points 5.99 / 1.61 / 1.07, at D=59, 128 dofs,
-// 16,384 points 30.0 / 16.2 / 16.0; F32 there 6.49 and 32.5 walking.
+// forming the split operands, and operands have 24 bits, as BF16X3's, where
+// F16X2's have 22. Measured (ms, walking / split operands in a direct sweep /
+// F32): F16X2 at D=24, 128 dofs, 30,011 points 5.99 / 1.61 / 1.07, at D=59, 128
+// dofs, 16,384 points 30.0 / 16.2 / 15.6; F32 there 6.49 and 32.5 walking, BF16X3
+// 7.30 and 34.9. Error against FP64 over 30 states of 241 to 7,081 nodes, D=4 to
+// 59 (F32's over the split one's, median and worst): F16X2 rms 0.72, 1.08, largest
+// 0.93, 1.60; BF16X3, which folds its sums after 16 nodes and not 32, rms 0.93,
+// 1.55, largest 1.46, 2.76 (D=6); none above 2.6e-7 of a column's largest value.
 // It needs surpluses that F32 holds; states with a dof column whose largest
 // value lies outside 2^-100 .. 2^100 keep the walking sweeps, whose f16
 // operands are scaled by column.
