@@ -353,3 +353,110 @@ def test_adjoint_of_large_batches_in_few_dimensions(dim, n):
     # dS sums n terms of size B g: 1e-12 of the largest leaves room for any order
     for (a, b), tol in zip(zip(*got), (1e-10, 1e-12)):
         assert (a - b).abs().max() <= tol * b.abs().max()
+
+
+@pytest.mark.parametrize("power", [99, 101, 120, -99, -101, -120])
+def test_split_precision_outside_the_range_of_f32(power):
+    """A dof column whose largest value lies outside 2^-100 .. 2^100 sends F16X2 to
+    the walking sweeps, whose operands are scaled by column."""
+    import torch
+    ii, jj, lv, ix = hddm_lb.generate_grid(6, 3, 4, 0.0, 7, 0)
+    r = np.random.default_rng(5)
+    S = r.uniform(-1.0, 1.0, (len(ii), 5))
+    S[0, 2] = 1.0
+    S[:, 2] *= 2.0 ** power
+    X = hddm_lb.synthetic_points(100, 6, 9)
+    c = hddm_lb.Context(0)
+    c.upload_state(0, ii, jj, S)
+    x = torch.from_numpy(X).cuda()
+    y = torch.full((100, 5), np.nan, dtype=torch.float64, device="cuda")
+    print("power", power, flush=True)
+    c.forward(x, y, None, hddm_lb.F16X2)
+    torch.cuda.synchronize()
+    assert c.last_config()["waves"] == (12 if abs(power) < 100 else 4)
+    c.close()
+    yo = oracle.forward(ii, jj, S, X)
+    den = oracle.forward(ii, jj, np.ones((len(ii), 1)), X).max() * np.abs(S).max(axis=0)
+    assert (np.abs(y.cpu().numpy() - yo).max(axis=0) <= 1e-6 * den).all()
+
+
+# the second state's grid, and the waves of F32 forwards of both in one context
+MIXED = [("thirds", 4), ("deep", 8), ("many hats", 8), ("fitting", 12)]
+
+
+@pytest.mark.parametrize("kind,waves", MIXED, ids=lambda v: str(v))
+def test_states_of_mixed_kinds_in_one_context(kind, waves):
+    """What a context's sweep and adjoint are follows from all of its states."""
+    import torch
+    dim, dofs, n = 10, 12, 300
+    r = np.random.default_rng(8)
+    grids = [hddm_lb.generate_grid(dim, 2, 4, 0.3, 7, 800)[:2]]
+    if kind == "thirds":
+        ii, jj = (a.copy() for a in hddm_lb.generate_grid(dim, 2, 3, 0.0, 7, 0)[:2])
+        third = ii == 4
+        ii[third], jj[third] = 3, np.minimum(jj[third], 2)
+    elif kind == "deep":
+        ii = np.unique((r.random((300, dim)) < 0.8) * 2, axis=0).astype(np.int32)
+        jj = ii.copy()
+        assert (ii > 0).sum(1).max() >= 8
+    elif kind == "many hats":
+        ii, jj = hddm_lb.generate_grid(dim, 6, 7, 0.0, 7, 0)[:2]
+        rows = np.sort(r.choice(len(ii), 900, replace=False))
+        single = np.flatnonzero((ii > 0).sum(1) == 1)
+        rows = np.unique(np.concatenate([rows, single]))
+        ii, jj = np.ascontiguousarray(ii[rows]), np.ascontiguousarray(jj[rows])
+    else:
+        ii, jj = hddm_lb.generate_grid(dim, 2, 4, 0.3, 9, 500)[:2]
+    grids.append((ii, jj))
+    c = hddm_lb.Context(0)
+    states = []
+    for s, (i, j) in enumerate(grids):
+        S = r.standard_normal((len(i), dofs))
+        c.upload_state(s, i, j, S)
+        states.append((i, j, S))
+    X = hddm_lb.synthetic_points(n, dim, 9)
+    sid = r.integers(0, 2, n).astype(np.int32)
+    G = r.standard_normal((n, dofs))
+    x, t, g = torch.from_numpy(X).cuda(), torch.from_numpy(sid).cuda(), torch.from_numpy(G).cuda()
+    for prec, tol in ((hddm_lb.F32, 1e-6), (hddm_lb.FP64, 1e-12)):
+        y = torch.full((n, dofs), np.nan, dtype=torch.float64, device="cuda")
+        print(kind, "precision", prec, flush=True)
+        c.forward(x, y, t, prec)
+        torch.cuda.synchronize()
+        if prec == hddm_lb.F32:
+            assert c.last_config()["waves"] == waves
+        for s, (i, j, S) in enumerate(states):
+            den = oracle.forward(i, j, np.ones((len(i), 1)), X[sid == s]).max() * np.abs(S).max()
+            assert np.abs(y.cpu().numpy()[sid == s] - oracle.forward(i, j, S, X[sid == s])).max() <= tol * den
+    dx, ds = torch.full_like(x, np.nan), torch.full((c.surplus_offset(-1)[1],), np.nan, dtype=torch.float64, device="cuda")
+    c.adjoint(x, g, dx, ds, t, hddm_lb.FP64)
+    torch.cuda.synchronize()
+    for s, (i, j, S) in enumerate(states):
+        dxo, dso = oracle.adjoint(i, j, S, X[sid == s], G[sid == s])
+        at = c.surplus_offset(s)[0]
+        assert np.abs(dx.cpu().numpy()[sid == s] - dxo).max() <= 1e-10 * np.abs(dxo).max()
+        assert np.abs(ds.cpu().numpy()[at:at + S.size] - dso.reshape(-1)).max() <= 1e-12 * np.abs(dso).max()
+    c.close()
+
+
+@pytest.mark.parametrize("case", [(6, 3, 5, 0.0, 0, 17, 17, 64), (6, 3, 5, 0.0, 0, 65, 31, 65), (16, 2, 6, 0.3, 6000, 1009, 32, 700),
+                                  (17, 2, 5, 0.3, 4000, 1024, 5, 129), (32, 2, 5, 0.3, 4000, 1500, 32, 200)],
+                         ids=lambda c: "d%d-n%d-c%d-p%d" % (c[0], c[5], c[6], c[7]))
+def test_adjoint_of_node_subsets_against_the_oracle(case):
+    """dx and dS of states whose paths have prefixes that are no nodes, at the
+    edges of windows, blocks and tiles."""
+    dim, base, depth, p, nodes, pick, dofs, npts = case
+    r = np.random.default_rng(pick)
+    ii, jj, lv, ix = hddm_lb.generate_grid(dim, base, depth, p, 7, nodes)
+    rows = np.sort(r.choice(len(ii), min(pick, len(ii)), replace=False))
+    ii, jj = np.ascontiguousarray(ii[rows]), np.ascontiguousarray(jj[rows])
+    S, G = r.standard_normal((len(rows), dofs)), r.standard_normal((npts, dofs))
+    X = hddm_lb.synthetic_points(npts, dim, 9)
+    X[0] = 0.5
+    c = hddm_lb.Context(0)
+    c.upload_state(0, ii, jj, S)
+    dx, ds = adjoint(c, X, G)
+    c.close()
+    dxo, dso = oracle.adjoint(ii, jj, S, X, G)
+    assert np.abs(dx - dxo).max() <= 1e-10 * np.abs(dxo).max()
+    assert np.abs(ds - dso.reshape(-1)).max() <= 1e-12 * np.abs(dso).max()
