@@ -112,7 +112,7 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 	for (;;)
 	{
 		__syncthreads();
-		if (threadIdx.x == 0) *slot = (int64_t)atomicAdd(&a.hdr->counter, 1ull);
+		if (threadIdx.x == 0) { slot[0] = (int64_t)atomicAdd(&a.hdr->counter, 1ull); slot[1] = 0; }
 		__syncthreads();
 		const int64_t item = (int64_t)uniform64((uint64_t)*slot);
 		if (item >= ldc(&a.hdr->nitems)) break;
@@ -138,6 +138,7 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 			for (int d = wave; d < a.dim; d += kAW) X[d * kWave + lane] = xrow[d];
 			// upstream gradient, 0 past the block and past the dofs: half a
 			// row per 16 lanes
+			bool odd = false;
 			for (int p = 4 * wave + row; p < kWave; p += 4 * kAW)
 			{
 				const uint32_t op = (uint32_t)__shfl((int)orig, p, 64);
@@ -146,9 +147,12 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 				for (int h = 0; h < 2; h++)
 				{
 					const int c = 16 * h + col;
-					G[p * kGRow + c] = p < np && c < dofs ? grow[c] : 0.0;
+					const double v = p < np && c < dofs ? grow[c] : 0.0;
+					odd |= !(fabs(v) < __builtin_huge_val());
+					G[p * kGRow + c] = v;
 				}
 			}
+			if (!DS && odd) slot[1] = 1;
 		}
 		__syncthreads();
 		// The hats at the block's points, and the points inside their
@@ -182,6 +186,7 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 		}
 		__syncthreads();
 
+		const bool wild = !DS && uniform((int)slot[1]) != 0;          // a gradient of the block is infinite or no number
 		const int nwin = (ldc(&sd->nops) + kWin - 1) / kWin;
 		const int nseg = (int)ldc(&pl->nseg);
 		const int s0 = (int)((int64_t)nwin * seg / nseg), s1 = (int)((int64_t)nwin * (seg + 1) / nseg);
@@ -242,7 +247,6 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 				}
 				uint32_t iv = 0;   // infos by slot
 				if constexpr (!DS) iv = info[(rv & kTabRow) >> 9];
-				const uint64_t bare = __builtin_amdgcn_ballot_w64((rv & kTabPrefix) != 0u);   // slots without a surplus
 				// The hats above slot j, by depth in the lanes, as offsets of
 				// their rows; depth lanes count.
 				auto above = [&](int j, int& depth) -> uint32_t {
@@ -375,9 +379,10 @@ __device__ __forceinline__ void adjoint_table(const AdjointArgs& a, int hats_max
 #pragma unroll
 								for (int m = 0; m < 4; m++) v[k + m] *= b[m];
 							}
-							// Empty slots and prefixes that are no nodes add nothing: an
-							// infinite gradient times their zeros is no number.
-							if ((bare >> (j0 + 8 * h)) & 0xffu)
+							// Empty slots add nothing, nor do prefixes that are no nodes
+							// where a gradient is infinite: times their zeros it is no
+							// number.
+							if (slots - j0 < 8 * h + 8 || wild)
 							{
 #pragma unroll
 								for (int k = 8 * h; k < 8 * h + 8; k++) v[k] = r[k] & kTabPrefix ? 0.0 : v[k];

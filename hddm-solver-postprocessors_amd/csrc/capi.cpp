@@ -532,6 +532,7 @@ int prepare_tables(hddm_lb_ctx* ctx)
 	ctx->nseg_adj_total = 0;
 	ctx->direct_ok = true;
 	ctx->f32_range = true;
+	ctx->odd = false;
 	ctx->hats_max = kHatFirst;
 	int64_t ds_offset = 0;
 	for (int s = 0; s < ns; s++)
@@ -584,6 +585,7 @@ int prepare_tables(hddm_lb_ctx* ctx)
 		ctx->fmax_all = std::max(ctx->fmax_all, d.max_depth);
 		ctx->direct_ok = ctx->direct_ok && d.hats > 0;
 		ctx->f32_range = ctx->f32_range && d.f32_range;
+		ctx->odd = ctx->odd || d.odd;
 		ctx->hats_max = std::max(ctx->hats_max, d.hats);
 		ctx->centre_exact_all = ctx->centre_exact_all && slot.centre_exact;
 		if (d.nseg > 1) ctx->max_nseg_dp = std::max<int64_t>(ctx->max_nseg_dp, (int64_t)d.nseg * d.dofs_pad);
@@ -907,7 +909,7 @@ int enqueue_forward(hddm_lb_ctx* ctx, Scratch& sc, int64_t npoints, const double
 		HIP_TRY(launch_scatter(npoints, sc.bkey, sc.cursor, sc.perm, st));
 	}
 
-	const void* kern = table ? sweep_table_kernel_ptr(sweep_prec(prec)) : !walking ? sweep_direct_kernel_ptr(sweep_prec(prec))
+	const void* kern = table ? sweep_table_kernel_ptr(sweep_prec(prec)) : !walking ? sweep_direct_kernel_ptr(sweep_prec(prec), ctx->odd)
 		: cfg.ws ? sweep_ws_kernel_ptr(prec, xbanks_for(ctx->dim), ctx->fmax_all, cfg.nc)
 		: sweep_kernel_ptr(walk_prec, cfg.slab, xbanks_for(ctx->dim), ctx->fmax_all, cfg.walk);
 	if (!kern) return set_error(HDDM_LB_ERROR_INVALID_VALUE, "forward: no sweep kernel for precision %d, dim %d", prec, ctx->dim);

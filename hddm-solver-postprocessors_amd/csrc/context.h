@@ -142,6 +142,7 @@ struct hddm_lb_ctx
 	bool table_ok = false;       // and the hat-table sweep's limits hold
 	int hats_max = 0;            // most hat ids of a state
 	bool f32_range = false;      // every state's surpluses are in F32's range
+	bool odd = false;            // a state has surpluses that are infinite or no numbers
 	hddm_lb::StateDesc* d_states = nullptr;
 	// the same descriptors with the wave-specialized adjoint's segment tables
 	hddm_lb::StateDesc* d_states_adj = nullptr;

@@ -31,6 +31,7 @@ struct HatCount
 	int overflow;                         // a key found no slot, or there are more than kMaxHats
 	int wide;                             // a dof column's largest value is out of F32's range
 	int found;                            // keys inserted
+	int odd;                              // a surplus is infinite or no number
 };
 static_assert(sizeof(HatCount) <= kHatFirst * 16, "fits");
 
@@ -54,7 +55,7 @@ __global__ void rec_kernel(HatTable* __restrict__ t, HatCount* __restrict__ cnt,
 {
 	const int q = blockIdx.x * blockDim.x + threadIdx.x;
 	if (q < kHashSlots) t->key[q] = 0ull;
-	if (q == 0) *cnt = HatCount{ 0, 0, 0, 0 };
+	if (q == 0) *cnt = HatCount{ 0, 0, 0, 0, 0 };
 	if (q < npad - nno) { rec[2 * (nno + q)] = 0u; rec[2 * (nno + q) + 1] = 0xc0000000u; }
 	if (q >= nops) return;
 	const Op op = ops[q];
@@ -201,6 +202,14 @@ __global__ void table_rec_kernel(int nops, int npad, int hstride, const Op* __re
 		thid[(size_t)q * hstride + f] = q >= nops ? (uint16_t)(8 * kHatNone) : f <= t ? ids[f] : (uint16_t)(8 * kHatAll);
 }
 
+__global__ void odd_kernel(int64_t n, const double* __restrict__ s, HatCount* cnt)
+{
+	bool odd = false;
+	for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x)
+		odd |= !(fabs(s[k]) < __builtin_huge_val());
+	if (odd) cnt->odd = 1;
+}
+
 int grid_for(int64_t n) { return (int)((n + 255) / 256); }
 
 } // namespace
@@ -241,6 +250,8 @@ int build_direct_tables(StateDesc& d, bool centre_exact, const DeviceAlloc& allo
 	const int64_t nent = (int64_t)d.nno * fs;
 	hipLaunchKernelGGL(rec_kernel, dim3(grid_for(d.nops > kHashSlots ? d.nops : kHashSlots)), dim3(256), 0, st, t, cnt, d.nno, npad,
 		d.nops, d.ops, rec);
+	const int64_t nsur = (int64_t)d.nno * d.dofs_pad;
+	hipLaunchKernelGGL(odd_kernel, dim3(nsur < 2048 * 256 ? grid_for(nsur) : 2048), dim3(256), 0, st, nsur, d.s64, cnt);
 	hipLaunchKernelGGL(hat_insert_kernel, dim3(grid_for(nent)), dim3(256), 0, st, nent, d.ftab, t, cnt);
 	hipLaunchKernelGGL(prefix_kernel, dim3(grid_for((int64_t)d.nops * kWave)), dim3(256), 0, st, d.nno, d.nops, d.ops, rec);
 	hipLaunchKernelGGL(special_kernel, dim3(grid_for(npad / 8)), dim3(256), 0, st, d.nno, npad, rec);
@@ -248,7 +259,7 @@ int build_direct_tables(StateDesc& d, bool centre_exact, const DeviceAlloc& allo
 	hipLaunchKernelGGL(hat_lookup_kernel, dim3(grid_for((int64_t)npad * hs)), dim3(256), 0, st, d.nno, npad, fs, hs, d.ftab,
 		(const HatTable*)t, (const HatCount*)cnt, hid);
 	HIP_TRY(hipGetLastError());
-	HatCount found = { 0, 0, 0, 0 };
+	HatCount found = { 0, 0, 0, 0, 0 };
 	HIP_TRY(hipMemcpy(&found, cnt, sizeof(found), hipMemcpyDeviceToHost));
 	if (found.overflow || found.total > kMaxHats) { drop(base); return HDDM_LB_SUCCESS; }
 	if (found.total <= kMaxTableHats && d.max_depth <= kTabMaxFactors)
@@ -267,6 +278,7 @@ int build_direct_tables(StateDesc& d, bool centre_exact, const DeviceAlloc& allo
 	d.hat = hat;
 	d.hstride = hs;
 	d.f32_range = !found.wide;
+	d.odd = found.odd;
 	d.hats = found.total;
 	return HDDM_LB_SUCCESS;
 }

@@ -100,8 +100,9 @@ hipError_t launch_sweep(const void* kern, int grid, int waves, size_t lds, const
 // Dynamic LDS of the sweep: the workgroup's op tiles (kWalkLds), then per
 // wave the path stack and the chunk buffer.
 size_t sweep_lds_bytes(int prec, int waves, int depth, int walk);
-// Direct sweep (sweep_direct.hip): one wave per dof tile of the pass.
-const void* sweep_direct_kernel_ptr(int prec);
+// Direct sweep (sweep_direct.hip): one wave per dof tile of the pass. odd: a state
+// has infinite surpluses or ones that are no numbers.
+const void* sweep_direct_kernel_ptr(int prec, bool odd);
 size_t sweep_direct_lds_bytes(int dim, int hats_max);
 // Hat-table sweep (sweep_table.hip), FP64 and F32 (else NULL): four dof tiles
 // per launch, sweep_table_waves waves per workgroup, launched like the direct one.

@@ -81,6 +81,7 @@ struct StateDesc
 	// Tables of the direct sweep (direct_tables.hip); hats == 0: the state has
 	// none and runs on the walking sweeps.
 	int hats, hstride;              // entries of hat; 16-bit ids per node in hid (2, 4, 6, 8 or 16)
+	int odd;                        // a surplus is infinite or no number
 	int f32_range;                  // largest value of every dof column 0 or within 2^-100 .. 2^100
 	const uint32_t* rec;            // [nodes rounded up to 64][2], see kRec*
 	const uint16_t* hid;            // [nodes rounded up to 64][hstride] 8 x the hat of each factor
