@@ -109,9 +109,10 @@ __device__ __forceinline__ double hat(double x, double i, double nj)
 	return fmax(1.0 - fabs(fma(x, i, nj)), 0.0);
 }
 
-// A node that is not alive gets this for the high word of -j (-1e300): its
-// hat, and so its basis, is zero at every point.
-constexpr uint32_t kFarHigh = 0xfe37e43cu;
+// A node that is not alive gets this for the high word of -j, an infinity: its
+// hat, and so its basis, is zero at every point (a large number is met by a
+// coordinate as large).
+constexpr uint32_t kFarHigh = 0xfff00000u;
 
 // The contraction of a unit of eight nodes.
 template <int PREC> struct Contract;

@@ -460,3 +460,30 @@ def test_adjoint_of_node_subsets_against_the_oracle(case):
     dxo, dso = oracle.adjoint(ii, jj, S, X, G)
     assert np.abs(dx - dxo).max() <= 1e-10 * np.abs(dxo).max()
     assert np.abs(ds - dso.reshape(-1)).max() <= 1e-12 * np.abs(dso).max()
+
+
+def test_points_far_outside_meet_no_node_of_the_direct_sweep():
+    """No coordinate, however large, is inside the hat that stands for a dead
+    node's: 1e300-like values, infinities and NaN give the oracle's zeros."""
+    import torch
+    ii, jj, lv, ix = hddm_lb.generate_grid(4, 7, 8, 0.0, 7, 0)
+    S = np.random.default_rng(2).standard_normal((len(ii), 8))
+    far = np.array([0x7e37e43c << 32], np.uint64).view(np.float64)[0]
+    xs = [s * far / 2 ** k for k in range(9) for s in (1.0, -1.0)] + [np.inf, -np.inf, np.nan, 1e308]
+    X = np.full((4 * len(xs), 4), 0.3)
+    for d in range(4):
+        X[d * len(xs):(d + 1) * len(xs), d] = xs
+    # at these the hats of the dimension are zero, as they are just past the edge
+    Y = np.where(np.abs(X) < 1.0, X, 1.5)
+    yo = oracle.forward(ii, jj, S, Y)
+    c = hddm_lb.Context(0)
+    c.upload_state(0, ii, jj, S)
+    for prec, tol in ((hddm_lb.FP64, 1e-12), (hddm_lb.F32, 1e-6)):
+        for p in range(len(X)):
+            x = torch.from_numpy(X[p:p + 1]).cuda()
+            y = torch.zeros((1, 8), dtype=torch.float64, device="cuda")
+            c.forward(x, y, None, prec)
+            torch.cuda.synchronize()
+            assert c.last_config()["waves"] == 8
+            assert np.abs(y.cpu().numpy() - yo[p]).max() <= tol * np.abs(S).max() * 50, X[p]
+    c.close()
