@@ -90,7 +90,7 @@ __device__ __forceinline__ void plan_items(int nstates, const StateDesc* __restr
 		const int nseg = dnt ? sweep_nseg(states[s].nops, dnt, dg) : states[s].nseg;
 		plans[s].item_base = item;
 		plans[s].nseg = nseg;
-		item += (plans[s].nblk + group - 1) / group * nseg;
+		item += (int64_t)((plans[s].nblk + group - 1) / group) * nseg;
 		plans[s].partial_base = pbase;
 		plans[s].dx_base = xbase;
 		if (nseg > 1)
@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(1024) scan_plan_kernel(const uint32_t* __restr
 		int64_t hi = (int64_t)cursor[(int64_t)(s + 1) << bbits];
 		plans[s].start = lo;
 		plans[s].count = hi - lo;
-		plans[s].nblk = (hi - lo + kWave - 1) / kWave;
+		plans[s].nblk = (int)((hi - lo + kWave - 1) / kWave);
 	}
 	__syncthreads();
 	if (t == 0) plan_items(nstates, states, cost_order, plans, hdr, group, dxw, dnt, dg);
@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(1024) small_plan_kernel(int n, const double* _
 		const int64_t lo = h[s << bbits], hi = h[(s + 1) << bbits];
 		plans[s].start = lo;
 		plans[s].count = hi - lo;
-		plans[s].nblk = (hi - lo + kWave - 1) / kWave;
+		plans[s].nblk = (int)((hi - lo + kWave - 1) / kWave);
 	}
 	__syncthreads();
 	if (t == 0) plan_items(nstates, states, cost_order, plans, hdr, group, 0, dnt, dg);
@@ -675,7 +675,7 @@ __global__ void __launch_bounds__(256) reduce_partials_kernel(const StateDesc* _
 	double* __restrict__ y, int64_t ldy)
 {
 	const int s = blockIdx.y;
-	const int nseg = (int)plans[s].nseg;
+	const int nseg = plans[s].nseg;
 	if (nseg <= 1) return;
 	const int dofs = states[s].dofs, DP = states[s].dofs_pad;
 	const int64_t count = plans[s].count, start = plans[s].start;

@@ -143,12 +143,13 @@ struct StatePlan
 {
 	int64_t start;         // first sorted position of the state's points
 	int64_t count;         // number of points of the state
-	int64_t nblk;          // 64-point blocks
+	int nblk;              // 64-point blocks
+	int nseg;              // node segments of the state in this call
 	int64_t item_base;     // first work item (items ordered by state cost)
 	int64_t partial_base;  // element offset in the partial buffer (split states)
 	int64_t dx_base;       // element offset in the adjoint's dx partial buffer (split states)
-	int64_t nseg;          // node segments of the state in this call
 };
+static_assert(sizeof(StatePlan) == 48, "counts towards the scratch of the allocation-free forward");
 
 struct PlanHeader
 {

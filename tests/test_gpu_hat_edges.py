@@ -487,3 +487,33 @@ def test_points_far_outside_meet_no_node_of_the_direct_sweep():
             assert c.last_config()["waves"] == 8
             assert np.abs(y.cpu().numpy() - yo[p]).max() <= tol * np.abs(S).max() * 50, X[p]
     c.close()
+
+
+def test_allocation_free_forward_up_to_its_limit():
+    """The largest batch that five states' scratch leaves room for: 8 bytes a point,
+    the histogram, cursors and 48 bytes a state in 64 MiB. One more row of 32
+    points is refused."""
+    import torch
+    n = 8191936   # 2 (4 n + 4 * 6 * 2^15) + 256 + 256 = 2^26
+    assert 2 * (4 * n + 4 * 6 * 2 ** 15) + 512 == 2 ** 26
+    c = hddm_lb.Context(0)
+    ii = np.array([[0], [2], [2]], np.int32)
+    jj = np.array([[0], [0], [2]], np.int32)
+    S = np.array([[1.0], [2.0], [4.0]])
+    for s in range(5):
+        c.upload_state(s, ii, jj, (s + 1) * S)
+    x = torch.rand((n + 32, 1), dtype=torch.float64, device="cuda")
+    sid = torch.arange(n + 32, dtype=torch.int32, device="cuda") % 5
+    y = torch.full((n + 32, 1), np.nan, dtype=torch.float64, device="cuda")
+
+    def run(m):
+        return hddm_lb.lib.hddm_lb_forward_noalloc(c._h, m, x.data_ptr(), 1, sid.data_ptr(), y.data_ptr(), 1, hddm_lb.FP64, None)
+    torch.cuda.synchronize()
+    print("points", n, flush=True)
+    assert run(n) == 0, hddm_lb.last_error()
+    torch.cuda.synchronize()
+    t = x[:n, 0]
+    ref = (sid[:n] + 1) * (1.0 + 2.0 * (1.0 - 2.0 * t).clamp(min=0.0) + 4.0 * (2.0 * t - 1.0).clamp(min=0.0))
+    assert (y[:n, 0] - ref).abs().max() <= 1e-12 * 25
+    assert run(n + 32) != 0
+    c.close()
